@@ -61,7 +61,7 @@ int qs_qrow_dequant_rows(const int8_t* codes, const float* scales, int64_t N, in
  *   x_dtype F32 : W in fp32, fp32 accumulate, y F32 (QStore fp32 compute contract).
  *   x_dtype BF16: W rounded to bf16 per element, fp32 accumulate, y BF16 (W8A16).
  *   x_dtype F16 : W rounded to fp16 per element, fp32 accumulate, y F16.
- * M <= 2 (decode) and fp32 use a VALU kernel, larger M an MFMA kernel; results agree
+ * Few rows (decode) and fp32 use a VALU kernel, more rows an MFMA kernel; results agree
  * within the fp32-accumulation tolerance but are not bitwise batch invariant. */
 int qs_qrow_matmul(const void* x, int x_dtype, int64_t ldx, const int8_t* codes,
                    const float* scales, void* y, int64_t ldy, int64_t M, int64_t N,
@@ -101,6 +101,26 @@ int qs_qrow_matmul_batched(const void* x, int x_dtype, int64_t ldx, int n_linear
                            void* const* y, const int64_t* ldy, const int64_t* N, int64_t M,
                            int64_t K, void* workspace, size_t workspace_bytes, void* stream);
 int qs_qrow_swiglu_batched(const void* x, int64_t ldx, const int8_t* gate_codes,
+                           const float* gate_scales, const int8_t* up_codes,
+                           const float* up_scales, void* y, int64_t ldy, int64_t M, int64_t N,
+                           int64_t K, void* workspace, size_t workspace_bytes, void* stream);
+
+/* Many activation rows (prefill): the contracts of qs_qrow_matmul_multi for BF16 / F16 x and
+ * of qs_qrow_swiglu in one launch over all M rows.  K % 64 == 0 and 16-byte aligned
+ * activation and weight rows, otherwise QS_ERR_UNSUPPORTED.  The tile shape and the number
+ * of K slices follow (M, N, K); the slices' fp32 partial sums are added in slice order.
+ * qs_qrow_matmul, qs_qrow_matmul_multi and qs_qrow_swiglu take the same kernel above 32
+ * rows, without a K split.
+ *   workspace: qs_qrow_prefill_workspace_bytes(M, n_linear, N, K, swiglu) bytes, 16-byte
+ *              aligned (0: K is not split; null also asks for no split), contents
+ *              clobbered; calls that run concurrently need their own. */
+size_t qs_qrow_prefill_workspace_bytes(int64_t M, int n_linear, const int64_t* N, int64_t K,
+                                       int swiglu);
+int qs_qrow_matmul_prefill(const void* x, int x_dtype, int64_t ldx, int n_linear,
+                           const int8_t* const* codes, const float* const* scales,
+                           void* const* y, const int64_t* ldy, const int64_t* N, int64_t M,
+                           int64_t K, void* workspace, size_t workspace_bytes, void* stream);
+int qs_qrow_swiglu_prefill(const void* x, int64_t ldx, const int8_t* gate_codes,
                            const float* gate_scales, const int8_t* up_codes,
                            const float* up_scales, void* y, int64_t ldy, int64_t M, int64_t N,
                            int64_t K, void* workspace, size_t workspace_bytes, void* stream);

@@ -14,7 +14,7 @@
 // MFMA operand mapping (16x16x32, wave64): lane l supplies row (l & 15) of A and column
 // (l & 15) of B, 8 consecutive k of k-block (l >> 4); the accumulator of lane l holds
 // D[4(l >> 4) + q][l & 15], q = 0..3.
-#include "qs_common.h"
+#include "qs_w8a16.h"
 
 #include <algorithm>
 
@@ -40,42 +40,6 @@ struct BdecParams {
   BdecLin lin[4];
   bool f16;
 };
-
-template <bool F16>
-struct Half;
-template <>
-struct Half<false> {
-  typedef bf16x8 vec;
-  static __device__ __forceinline__ void deq(i32x4 w, float s, vec& lo, vec& hi) { deq16_bf16(w, s, lo, hi); }
-  static __device__ __forceinline__ f32x4 mma(vec a, vec b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t out(float v) { return f32_to_bf16_bits(v); }
-};
-template <>
-struct Half<true> {
-  typedef f16x8 vec;
-  static __device__ __forceinline__ void deq(i32x4 w, float s, vec& lo, vec& hi) { deq16_f16(w, s, lo, hi); }
-  static __device__ __forceinline__ f32x4 mma(vec a, vec b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t out(float v) { return f32_to_f16_bits(v); }
-};
-
-__device__ __forceinline__ float silu(float g) { return g * (1.0f / (1.0f + expf(-g))); }
-
-// Epilogue of one output: plane sums -> bf16/f16 (P = 1) or the paired SwiGLU (P = 2).
-template <int P, bool F16>
-__device__ __forceinline__ uint16_t bdec_out(const float (&v)[P]) {
-  if constexpr (P == 2) {
-    const float gt = bf16_bits_to_f32(f32_to_bf16_bits(v[0]));
-    const float ut = bf16_bits_to_f32(f32_to_bf16_bits(v[1]));
-    const float sl = bf16_bits_to_f32(f32_to_bf16_bits(silu(gt)));
-    return f32_to_bf16_bits(sl * ut);
-  } else {
-    return Half<F16>::out(v[0]);
-  }
-}
 
 int bdec_prepare(BdecParams& p, const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K) {
   if (!x) return fail(QS_ERR_INVALID, "qrow batched: null activations");
@@ -184,7 +148,7 @@ __device__ __forceinline__ void bd2_finish(const Bd2Params& p, const BdecLin& L0
         float v[P];
 #pragma unroll
         for (int pl = 0; pl < P; ++pl) v[pl] = out[pl][t][q];
-        o[q] = bdec_out<P, F16>(v);
+        o[q] = w8a16_out<P, F16>(v);
       }
       uint16_t* yr = y + (int64_t)m * L0.ldy + nb;
       if (full) {
@@ -410,7 +374,7 @@ __global__ __launch_bounds__(128) void k_bd2_reduce(Bd2Params p) {
     float v[P];
 #pragma unroll
     for (int pl = 0; pl < P; ++pl) v[pl] = a[pl][q];
-    o[q] = bdec_out<P, F16>(v);
+    o[q] = w8a16_out<P, F16>(v);
   }
   uint16_t* yr = static_cast<uint16_t*>(L.y) + (int64_t)m * L.ldy + (ncol - L.n_begin);
   if (p.vec) {

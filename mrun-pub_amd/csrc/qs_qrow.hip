@@ -40,7 +40,7 @@
 // 32 contiguous bytes at k = 128*c + 32*(l>>4) of weight row (l & 15) and the matching
 // 32 activations; each 8 of them feed one MFMA (4 per 128-k chunk).  The accumulator of
 // lane l holds D[4*(l>>4) + q][l & 15], q = 0..3.
-#include "qs_common.h"
+#include "qs_w8a16.h"
 
 #include <mutex>
 #include <type_traits>
@@ -1768,13 +1768,20 @@ void launch_top2_mb(const QrowParams& q, int rows, int start_row, float* pv, int
 // blocks; the fused path uses 8-row blocks, so this bounds both).
 int64_t top2_blocks(int64_t rows) { return cdiv(rows, 4); }
 
-// Runs one set of linears sharing x, M <= 32 rows at a time for the MFMA path.
+// Runs one set of linears sharing x.
 int run_linears(QrowParams p, int x_dtype, int64_t M, hipStream_t s, bool row_stable) {
   if (M == 0) return QS_OK;
   const int esz = x_dtype == QS_F32 ? 4 : 2;
   // decode-sized batches (and the row-stable contract) take the VALU path
   if ((row_stable || M <= kValuRows || x_dtype == QS_F32) && valu_eligible(p, x_dtype))
     return run_valu(p, x_dtype, M, s, false);
+  if (!row_stable && M > 32 && x_dtype != QS_F32) {  // one launch for all rows (qs_prefill.hip)
+    QrowPrefillLin lin[4];
+    for (int i = 0; i < p.n_lin; ++i)
+      lin[i] = QrowPrefillLin{p.lin[i].codes, p.lin[i].scales, p.lin[i].y, p.lin[i].ldy, p.lin[i].N};
+    const int st = run_prefill(p.x, x_dtype == QS_F16, p.ldx, p.n_lin, lin, 1, M, p.K, nullptr, 0, s);
+    if (st != QS_ERR_UNSUPPORTED) return st;
+  }
   if (!row_stable && mfma_eligible(p, x_dtype)) {
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
       QrowParams q = p;
@@ -1935,6 +1942,11 @@ extern "C" int qs_qrow_swiglu(const void* x, int64_t ldx, const int8_t* gate_cod
   p.lin[0] = QrowLin{gate_codes, gate_scales, y, ldy, (int)N, 0};
   p.lin[1] = QrowLin{up_codes, up_scales, nullptr, 0, (int)N, 0};
   if (M <= kValuRows && valu_eligible(p, QS_BF16)) return run_valu(p, QS_BF16, M, s, true);
+  if (M > 32) {
+    const QrowPrefillLin lin[2] = {{gate_codes, gate_scales, y, ldy, N}, {up_codes, up_scales, nullptr, 0, N}};
+    st = run_prefill(x, false, ldx, 2, lin, 2, M, K, nullptr, 0, s);
+    if (st != QS_ERR_UNSUPPORTED) return st;
+  }
   if (mfma_eligible(p, QS_BF16)) {
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
       QrowParams q = p;

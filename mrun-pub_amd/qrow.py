@@ -140,7 +140,7 @@ def _out_buffer(out: torch.Tensor | None, m: int, n: int, dtype: torch.dtype, de
 
 # The batched kernels (k_bd2: an LDS activation slice shared by a workgroup's weight rows,
 # weights streamed into VGPRs, K split only for rows longer than 2048) serve every
-# bf16/f16 call with at least 16 activation rows: in same-box A/B timings of the config-2
+# bf16/f16 call with 16 to 32 activation rows: in same-box A/B timings of the config-2
 # shapes they match or beat the 16-row-tile kernels at M = 16 and beat them at M = 32
 # (1536 x 8960: 25.4 -> 11.5 us, paired SwiGLU 8960 x 1536: 18.5 -> 14.3 us).
 # Fewer rows take them where they measured faster than the 16-row-tile kernels that serve
@@ -149,7 +149,11 @@ def _out_buffer(out: torch.Tensor | None, m: int, n: int, dtype: torch.dtype, de
 # 9.9 us at M = 8, 15.2 -> 10.1 at M = 12); short rows keep the tiles below 16 (1536 x 1536
 # at M = 12: 4.89 against 5.03 us).  M <= 4 stays on the register-activation GEMV, whose
 # rows equal single-row results bit for bit (and whose chained M = 4 pass is faster).
+# Above 32 rows the prefill kernel (qs_prefill.hip) takes the whole call: at 33 rows one of
+# its launches (q/k/v 9.3 us, paired SwiGLU 15.1, 1536 x 8960 15.0) replaces two batched ones
+# (11, 23, 20), and 32-row batches would read the weights once per batch.
 BATCHED_MIN_M = 16
+BATCHED_MAX_M = 32
 BATCHED_MIN_M_SWIGLU = 5
 BATCHED_MIN_M_LONG = 8
 BATCHED_MAX_K = 16384
@@ -160,35 +164,51 @@ def _batched_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool 
     ns = [int(c.shape[0]) for c in codes]
     min_m = BATCHED_MIN_M_SWIGLU if swiglu else (BATCHED_MIN_M_LONG if k > 2048 else BATCHED_MIN_M)
     return (x2.dtype in (torch.bfloat16, torch.float16) and (not swiglu or x2.dtype == torch.bfloat16)
-            and m >= min_m and k % 128 == 0 and k <= BATCHED_MAX_K
+            and min_m <= m <= BATCHED_MAX_M and k % 128 == 0 and k <= BATCHED_MAX_K
             and (k <= 2048 or all(n % 4 == 0 for n in ns))
             and x2.stride(0) == k and x2.data_ptr() % 16 == 0 and all(c.data_ptr() % 16 == 0 for c in codes))
 
 
-def _run_batched(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
-                 swiglu: bool) -> None:
-    """``qs_qrow_matmul_batched`` / ``qs_qrow_swiglu_batched`` over row batches of <= 32,
-    with a workspace for the K-slice partial sums (the split depends on N and K only)."""
+def _prefill_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool = False) -> bool:
+    """More rows than a batch, in the layout qs_qrow_matmul_prefill takes (rows of whole 64-k
+    steps, 16-byte aligned; the offsets inside a 128-row tile are 31-bit)."""
+    m, k = int(x2.shape[0]), int(x2.shape[1])
+    return (m > BATCHED_MAX_M and x2.dtype in (torch.bfloat16, torch.float16)
+            and (not swiglu or x2.dtype == torch.bfloat16) and k % 64 == 0 and k < 1 << 22
+            and x2.stride(0) == k and x2.data_ptr() % 16 == 0 and all(c.data_ptr() % 16 == 0 for c in codes))
+
+
+def _run_many(kind: str, x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
+              swiglu: bool) -> None:
+    """``qs_qrow_matmul_<kind>`` / ``qs_qrow_swiglu_<kind>`` (kind: batched or prefill) with a
+    workspace for the K-slice partial sums."""
     device = x2.device
-    m_all, k = int(x2.shape[0]), int(x2.shape[1])
+    m, k = int(x2.shape[0]), int(x2.shape[1])
     ns = [int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]]
     stream = nat.stream_of(device)
     n_arr = nat.int64_array(ns)
-    lib = nat.load()
-    ws_bytes = int(lib.qs_qrow_batched_workspace_bytes(min(32, m_all), len(ns), n_arr, k, int(swiglu)))
+    ws_bytes = int(getattr(nat.load(), f"qs_qrow_{kind}_workspace_bytes")(m, len(ns), n_arr, k, int(swiglu)))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=device)
-    for m0 in range(0, m_all, 32):
-        mm = min(32, m_all - m0)
-        xb = x2[m0:m0 + mm]
-        if swiglu:
-            (gc, gs), (uc, us) = pages
-            nat.call("qs_qrow_swiglu_batched", nat.ptr(xb), k, nat.ptr(gc), nat.ptr(gs), nat.ptr(uc), nat.ptr(us),
-                     nat.ptr(outs[0][m0:]), ns[0], mm, ns[0], k, nat.ptr(ws), ws_bytes, stream)
-        else:
-            nat.call("qs_qrow_matmul_batched", nat.ptr(xb), nat.dtype_code(x2.dtype), k, len(pages),
-                     nat.pointer_array([nat.ptr(c) for c, _ in pages]), nat.pointer_array([nat.ptr(sc) for _, sc in pages]),
-                     nat.pointer_array([nat.ptr(o[m0:]) for o in outs]), n_arr, n_arr, mm, k, nat.ptr(ws), ws_bytes,
-                     stream)
+    if swiglu:
+        (gc, gs), (uc, us) = pages
+        nat.call(f"qs_qrow_swiglu_{kind}", nat.ptr(x2), k, nat.ptr(gc), nat.ptr(gs), nat.ptr(uc), nat.ptr(us),
+                 nat.ptr(outs[0]), ns[0], m, ns[0], k, nat.ptr(ws), ws_bytes, stream)
+    else:
+        nat.call(f"qs_qrow_matmul_{kind}", nat.ptr(x2), nat.dtype_code(x2.dtype), k, len(pages),
+                 nat.pointer_array([nat.ptr(c) for c, _ in pages]), nat.pointer_array([nat.ptr(sc) for _, sc in pages]),
+                 nat.pointer_array([nat.ptr(o) for o in outs]), n_arr, n_arr, m, k, nat.ptr(ws), ws_bytes, stream)
+
+
+def _run_batched(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
+                 swiglu: bool) -> None:
+    """At most 32 rows through the batched kernels (the split depends on N and K only)."""
+    _run_many("batched", x2, pages, outs, swiglu)
+
+
+def _run_prefill(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
+                 swiglu: bool) -> None:
+    """Any number of rows through the prefill kernel."""
+    _run_many("prefill", x2, pages, outs, swiglu)
 
 
 @torch.inference_mode()
@@ -218,6 +238,8 @@ def qrow_matmul(
     y = _out_buffer(out, m, n, x.dtype, device)
     if m and not row_stable and _batched_eligible(flat, [codes]):
         _run_batched(flat, [(codes, scales)], [y], swiglu=False)
+    elif m and not row_stable and _prefill_eligible(flat, [codes]):
+        _run_prefill(flat, [(codes, scales)], [y], swiglu=False)
     elif m:
         nat.call(
             "qs_qrow_matmul_row_stable" if row_stable else "qs_qrow_matmul",
@@ -259,6 +281,8 @@ def qrow_matmul_multi(
     outs = [_out_buffer(None if out is None else out[i], m, n, x.dtype, device) for i, (n, _) in enumerate(shapes)]
     if m and _batched_eligible(flat, [c for c, _ in pages]):
         _run_batched(flat, pages, outs, swiglu=False)
+    elif m and _prefill_eligible(flat, [c for c, _ in pages]):
+        _run_prefill(flat, pages, outs, swiglu=False)
     elif m:
         nat.call(
             "qs_qrow_matmul_multi",
@@ -356,6 +380,8 @@ def qrow_swiglu_into(gate_page: CompactQRowPage, up_page: CompactQRowPage, activ
     y = _out_buffer(out, m, n, torch.bfloat16, device)
     if m and _batched_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
         _run_batched(flat, [(gate_page.codes, gate_page.scales), (up_page.codes, up_page.scales)], [y], swiglu=True)
+    elif m and _prefill_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
+        _run_prefill(flat, [(gate_page.codes, gate_page.scales), (up_page.codes, up_page.scales)], [y], swiglu=True)
     elif m:
         nat.call(
             "qs_qrow_swiglu",

@@ -1,0 +1,120 @@
+"""GPU parity of the many-row (prefill) W8A16 kernels against the CPU oracle."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import qrow as oq
+
+pytestmark = pytest.mark.gpu
+
+# The oracle rounds the same sums once to 16 bits.  fp32 sums of at most 8960 products in
+# another order move a sum by about 1e-6 of its terms' norm, which flips the rounding of
+# roughly 1 output in 4000 by one ulp (2^-8 / 2^-11 relative): rel-L2 below 1e-4.
+TOL = 1e-3
+
+
+def _case(n, k, seed):
+    rng = np.random.default_rng(seed)
+    codes = rng.integers(-127, 128, size=(n, k), dtype=np.int8)
+    scales = (rng.uniform(0.5, 1.5, size=n) / 127).astype(np.float32)
+    return codes, scales
+
+
+def _x(m, k, seed, f16):
+    x = np.random.default_rng(seed).standard_normal((m, k)).astype(np.float32)
+    return oq.round_f16(x) if f16 else oq.round_bf16(x)
+
+
+def _guarded(m, n, dtype, dev):
+    """A contiguous [m, n] output between 256 sentinel elements on both sides."""
+    buf = torch.full((m * n + 512,), 7.0, dtype=dtype, device=dev)
+    return buf, buf[256:256 + m * n].view(m, n)
+
+
+def _untouched(buf, m, n):
+    return bool((buf[:256] == 7).all()) and bool((buf[256 + m * n:] == 7).all())
+
+
+# Tile edges (16/32/64/128 activation rows, 128 weight rows), ragged N (N % 4 != 0 also turns
+# the K split and the vector stores off), one to a few K steps, and K splits.
+@pytest.mark.parametrize("m", [33, 64, 65, 129, 300])
+@pytest.mark.parametrize("n,k", [(5, 64), (127, 128), (129, 320), (256, 1536), (72, 8960), (1030, 1088)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_prefill_matmul(dev, m, n, k, f16):
+    from mrun_pub_amd import qrow as q
+
+    codes, scales = _case(n, k, seed=m + n + k)
+    x = _x(m, k, m + k, f16)
+    dt = torch.float16 if f16 else torch.bfloat16
+    c, s, xd = torch.from_numpy(codes).to(dev), torch.from_numpy(scales).to(dev), torch.from_numpy(x).to(dev).to(dt)
+    assert q._prefill_eligible(xd, [c])
+    buf, out = _guarded(m, n, dt, dev)
+    y = q.qrow_matmul(c, s, xd, out=out)
+    ref = oq.qrow_matmul_w8a16(codes, scales, x, "fp16" if f16 else "bf16")
+    assert oq.rel_l2(y.float().cpu().numpy(), ref) <= TOL
+    assert _untouched(buf, m, n)
+    # without a workspace (no K split): the entry points that take none
+    buf, out = _guarded(m, n, dt, dev)
+    q.nat.call("qs_qrow_matmul", xd.data_ptr(), q.nat.dtype_code(dt), k, c.data_ptr(), s.data_ptr(), out.data_ptr(), n,
+               m, n, k, q.nat.stream_of(dev))
+    assert oq.rel_l2(out.float().cpu().numpy(), ref) <= TOL
+    assert _untouched(buf, m, n)
+
+
+@pytest.mark.parametrize("m", [33, 100, 200])
+@pytest.mark.parametrize("n,k", [(7, 64), (64, 1024), (200, 384), (68, 4096)])
+def test_prefill_swiglu(dev, m, n, k):
+    from mrun_pub_amd import qrow as q
+
+    g, u = _case(n, k, seed=m + n), _case(n, k, seed=m + n + 1)
+    x = _x(m, k, m + k, False)
+    xd = torch.from_numpy(x).to(dev).to(torch.bfloat16)
+    pages = [q.CompactQRowPage(nm, 0, n, k, torch.from_numpy(w[0]).to(dev), torch.from_numpy(w[1]).to(dev))
+             for nm, w in (("g", g), ("u", u))]
+    buf, out = _guarded(m, n, torch.bfloat16, dev)
+    y = q.qrow_swiglu_into(pages[0], pages[1], xd, out)
+    ref = oq.qrow_swiglu(*g, *u, x)
+    # a flipped gate or up rounding is one ulp of the product too: the same bar
+    assert oq.rel_l2(y.float().cpu().numpy(), ref) <= TOL
+    assert _untouched(buf, m, n)
+    buf, out = _guarded(m, n, torch.bfloat16, dev)
+    q.nat.call("qs_qrow_swiglu", xd.data_ptr(), k, *(t.data_ptr() for p in pages for t in (p.codes, p.scales)),
+               out.data_ptr(), n, m, n, k, q.nat.stream_of(dev))
+    assert oq.rel_l2(out.float().cpu().numpy(), ref) <= TOL
+    assert _untouched(buf, m, n)
+
+
+@pytest.mark.parametrize("m", [40, 333])
+@pytest.mark.parametrize("ns", [[1536, 256, 256], [130, 3], [64, 128, 16, 4]])
+def test_prefill_multi_equals_oracle(dev, m, ns):
+    """Linears of different widths in one launch, each with its own tiles."""
+    from mrun_pub_amd import qrow as q
+
+    k = 1536
+    ws = [_case(n, k, seed=n + i) for i, n in enumerate(ns)]
+    x = _x(m, k, m, False)
+    xd = torch.from_numpy(x).to(dev).to(torch.bfloat16)
+    bufs, outs = zip(*(_guarded(m, n, torch.bfloat16, dev) for n in ns))
+    q.qrow_matmul_multi([(torch.from_numpy(c).to(dev), torch.from_numpy(s).to(dev)) for c, s in ws], xd, out=list(outs))
+    for (c, s), n, y, buf in zip(ws, ns, outs, bufs):
+        assert oq.rel_l2(y.float().cpu().numpy(), oq.qrow_matmul_w8a16(c, s, x)) <= TOL
+        assert _untouched(buf, m, n)
+
+
+def test_prefill_nonfinite_stays_in_its_row(dev):
+    """An infinity or NaN in one activation row reaches that row only."""
+    from mrun_pub_amd import qrow as q
+
+    n, k, m = 136, 256, 70
+    codes, scales = _case(n, k, seed=3)
+    x = _x(m, k, 4, False)
+    x[5, 17] = np.inf
+    x[69, 0] = np.nan
+    y = q.qrow_matmul(torch.from_numpy(codes).to(dev), torch.from_numpy(scales).to(dev),
+                      torch.from_numpy(x).to(dev).to(torch.bfloat16)).float().cpu().numpy()
+    rows = np.array([r for r in range(m) if r not in (5, 69)])
+    assert np.isfinite(y[rows]).all() and not np.isfinite(y[5]).any() and np.isnan(y[69]).all()
+    assert oq.rel_l2(y[rows], oq.qrow_matmul_w8a16(codes, scales, x[rows])) <= TOL
