@@ -105,17 +105,17 @@ int qs_qrow_swiglu_batched(const void* x, int64_t ldx, const int8_t* gate_codes,
                            const float* up_scales, void* y, int64_t ldy, int64_t M, int64_t N,
                            int64_t K, void* workspace, size_t workspace_bytes, void* stream);
 
-/* Many activation rows (prefill): the contracts of qs_qrow_matmul_multi for BF16 / F16 x and
- * of qs_qrow_swiglu in one launch over all M rows.  K % 64 == 0 and 16-byte aligned
+/* Many activation rows (prefill): the contracts of qs_qrow_matmul_multi and of
+ * qs_qrow_swiglu in one launch over all M rows.  K % 64 == 0 and 16-byte aligned
  * activation and weight rows, otherwise QS_ERR_UNSUPPORTED.  The tile shape and the number
  * of K slices follow (M, N, K); the slices' fp32 partial sums are added in slice order.
- * qs_qrow_matmul, qs_qrow_matmul_multi and qs_qrow_swiglu take the same kernel above 32
- * rows, without a K split.
- *   workspace: qs_qrow_prefill_workspace_bytes(M, n_linear, N, K, swiglu) bytes, 16-byte
- *              aligned (0: K is not split; null also asks for no split), contents
+ * qs_qrow_matmul, qs_qrow_matmul_multi and qs_qrow_swiglu take the same kernel, without a
+ * K split, above 32 rows of BF16 / F16 and for batches of more than a few F32 rows.
+ *   workspace: qs_qrow_prefill_workspace_bytes(x_dtype, M, n_linear, N, K, swiglu) bytes,
+ *              16-byte aligned (0: K is not split; null also asks for no split), contents
  *              clobbered; calls that run concurrently need their own. */
-size_t qs_qrow_prefill_workspace_bytes(int64_t M, int n_linear, const int64_t* N, int64_t K,
-                                       int swiglu);
+size_t qs_qrow_prefill_workspace_bytes(int x_dtype, int64_t M, int n_linear, const int64_t* N,
+                                       int64_t K, int swiglu);
 int qs_qrow_matmul_prefill(const void* x, int x_dtype, int64_t ldx, int n_linear,
                            const int8_t* const* codes, const float* const* scales,
                            void* const* y, const int64_t* ldy, const int64_t* N, int64_t M,

@@ -1,10 +1,10 @@
-// W8A16 qrow linears for many activation rows (prefill) on gfx950.
+// qrow linears for many activation rows (prefill) on gfx950: W8A16 and fp32.
 //
 // Kernels
-//   k_prefill<P, MT, NT, WN, WK, D, F16> : one workgroup = a tile of 16 * MT activation rows
+//   k_prefill<P, MT, NT, WN, WK, D, XT> : one workgroup = a tile of 16 * MT activation rows
 //                               and 16 * NT * WN weight rows (of P planes; P = 2 pairs the
 //                               gate and up rows of a SwiGLU) x one K slice.
-//   k_prefill_reduce<P, F16>  : the K slices' fp32 partial sums added in slice order, and the
+//   k_prefill_reduce<P, XT>   : the K slices' fp32 partial sums added in slice order, and the
 //                               epilogue.
 #include "qs_w8a16.h"
 
@@ -26,7 +26,7 @@ struct PfLin {
 };
 
 struct PfParams {
-  const uint16_t* x;
+  const void* x;
   int64_t ldx;
   int M, K;
   int T, TS;  // 64-k steps, and steps per slice
@@ -79,16 +79,27 @@ constexpr int kPfFlush = 6;
 // phases of a CU's two or three workgroups overlap only in part.  Pinning the conversions
 // between the MFMAs (one pair of codes per two MFMAs) was 10% slower, as was a third group in
 // flight.
-template <int P, int MT, int NT, int WN, int WK, int D, bool F16>
+//
+// fp32 activations run on v_mfma_f32_16x16x4 (a sixteenth of the bf16 rate), so there the
+// matrix pipe is the bound and the tiles are small (16 or 32 rows) to keep every CU's busy:
+// 149 x 1536 x 8960 787 -> 54 us (75 TFLOP/s of the 135 that a 4096^3 library product reaches;
+// before: one launch of the one-row VALU kernel per row), 64 x 8960 x 1536 155 -> 29 us,
+// 9 x 4096 x 1024 15.0 -> 8.4 us.  Error against 64-bit sums 1.0e-7..1.2e-7 (VALU: 1.0e-7 at
+// K = 1024 to 2.3e-7 at K = 8960).
+template <int P, int MT, int NT, int WN, int WK, int D, int XT>
 __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
-  typedef Half<F16> H;
+  constexpr bool F32 = XT == QS_F32;
+  typedef Half<XT == QS_F16> H;
   typedef typename H::vec hvec;
   constexpr int NW = WN * WK;
   constexpr int TM = 16 * MT, TN = 16 * NT * WN;
-  constexpr int SUB = TM * 128;    // bytes of one 64-k step's activations
+  constexpr int ES = F32 ? 4 : 2;
+  constexpr int ROW = 64 * ES;     // bytes of one activation row's 64-k step
+  constexpr int SL = ROW / 16;     // its 16-byte chunks
+  constexpr int SUB = TM * ROW;    // bytes of one 64-k step's activations
   constexpr int STAGE = SUB * WK;
-  constexpr int XD = 2 * MT * WK / NW;  // 1 KiB copies per wave per stage
-  static_assert(XD * NW == 2 * MT * WK, "whole copies per wave");
+  constexpr int XD = STAGE / 1024 / NW;  // 1 KiB copies per wave per stage
+  static_assert(XD * NW * 1024 == STAGE, "whole copies per wave");
   constexpr int RED = WK > 1 ? (WK - 1) * WN * MT * 64 * 16 : 0;
   constexpr int LDS = (D + 1) * STAGE > RED ? (D + 1) * STAGE : RED;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS];
@@ -134,9 +145,9 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
   // operands through buffers that start at the tile's first row: rows past the operand and
   // steps past the slice read out of range (zero, no memory access)
   const int xrows = min(TM, p.M - bm);
-  const int xlim = (int)(((int64_t)(xrows - 1) * p.ldx + K) * 2);
+  const int xlim = (int)(((int64_t)(xrows - 1) * p.ldx + K) * ES);
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.x + (int64_t)bm * p.ldx), (short)0, xlim, 0x00020000);
+      const_cast<char*>(static_cast<const char*>(p.x) + (int64_t)bm * p.ldx * ES), (short)0, xlim, 0x00020000);
   const int wlim = min(TN, N - tb) * K;
   __amdgpu_buffer_rsrc_t wr[P];
 #pragma unroll
@@ -144,23 +155,24 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
     wr[pl] = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(p.lin[P == 2 ? pl : li].codes + (int64_t)tb * K), (short)0, wlim, 0x00020000);
 
-  // copy e of a stage: 8 rows x 128 bytes of sub-step e / (2 MT); lane l lands in row l >> 3,
-  // slot l & 7, which holds 16-byte chunk slot ^ ((row >> 1) & 7) (the 16 rows a fragment
-  // pass reads then fall in distinct bank groups)
+  // copy e of a stage: whole rows of one 64-k step; lane l lands in row l / SL, slot l % SL,
+  // which holds 16-byte chunk slot ^ (a hash of the row) (the 16 rows a fragment pass reads
+  // then fall in distinct bank groups)
+  auto swz = [](int r) { return F32 ? r & 15 : (r >> 1) & 7; };
   int xoff[XD], xsub[XD], xdst[XD];
 #pragma unroll
   for (int e = 0; e < XD; ++e) {
     const int c = wave * XD + e;
-    const int r = 8 * (c % (2 * MT)) + (lane >> 3);
-    xsub[e] = c / (2 * MT);
+    const int r = (64 / SL) * (c % (SUB / 1024)) + lane / SL;
+    xsub[e] = c / (SUB / 1024);
     xdst[e] = 1024 * c;
-    xoff[e] = r * (int)p.ldx * 2 + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+    xoff[e] = r * (int)p.ldx * ES + 16 * ((lane % SL) ^ swz(r));
   }
   auto copy_x = [&](int i, int st) {  // iteration i -> stage st
 #pragma unroll
     for (int e = 0; e < XD; ++e) {
       const int t = i * WK + xsub[e];
-      pf_copy16(xr, lds + st * STAGE + xdst[e], t < T ? xoff[e] : xlim, t < T ? (t0 + t) * 128 : 0);
+      pf_copy16(xr, lds + st * STAGE + xdst[e], t < T ? xoff[e] : xlim, t < T ? (t0 + t) * ROW : 0);
     }
   };
   const int wlane = (16 * NT * wn + col) * K + 16 * grp;
@@ -183,15 +195,16 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[pl][j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int sw = (col >> 1) & 7;
-  const int xr0 = col * 128 + 16 * ((2 * grp) ^ sw), xr1 = col * 128 + 16 * ((2 * grp + 1) ^ sw);
   // iteration i from stage st; its weight registers take the weights of iteration i + D as
-  // soon as they are dequantized
-  auto mul = [&](i32x4 (&w)[P][NT], int i, int st) {
-    const uint8_t* xs = lds + st * STAGE + wk * SUB;
+  // soon as they are dequantized.  16-bit: the lane's 16 codes make two MFMA fragments.
+  const int sw = swz(col);
+  auto mul16 = [&](i32x4 (&w)[P][NT], int i, int st) {
+    const uint8_t* xs = lds + st * STAGE + wk * SUB + col * ROW;
+    const uint8_t* x0 = xs + 16 * ((2 * grp) ^ sw);
+    const uint8_t* x1 = xs + 16 * ((2 * grp + 1) ^ sw);
     hvec xa[MT], xb[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) xa[m] = *reinterpret_cast<const hvec*>(xs + xr0 + 2048 * m);
+    for (int m = 0; m < MT; ++m) xa[m] = *reinterpret_cast<const hvec*>(x0 + 16 * ROW * m);
     hvec wb[P][NT][2];
 #pragma unroll
     for (int pl = 0; pl < P; ++pl)
@@ -205,13 +218,53 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[pl][j][m] = H::mma(wb[pl][j][0], xa[m], acc[pl][j][m]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) xb[m] = *reinterpret_cast<const hvec*>(xs + xr1 + 2048 * m);
+    for (int m = 0; m < MT; ++m) xb[m] = *reinterpret_cast<const hvec*>(x1 + 16 * ROW * m);
 #pragma unroll
     for (int pl = 0; pl < P; ++pl)
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[pl][j][m] = H::mma(wb[pl][j][1], xb[m], acc[pl][j][m]);
+  };
+  // fp32: each of the lane's 16 codes is one k of a 16x16x4 MFMA (four k per instruction, one
+  // from each lane group), weights float(code) * scale, products and sums in fp32.  Sums of 16
+  // k start from zero and the four of a step are added in pairs before they join the
+  // accumulators: short chains, as exact as the row's sum over a wave's lanes.
+  auto mul32 = [&](i32x4 (&w)[P][NT], int i, int st) {
+    const uint8_t* xs = lds + st * STAGE + wk * SUB + col * ROW;
+    i32x4 wv[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wv[j] = w[0][j];
+    load_w(w, i + D);
+    f32x4 part[2][NT][MT];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      f32x4 x[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) x[m] = *reinterpret_cast<const f32x4*>(xs + 16 * ((4 * grp + c) ^ sw) + 16 * ROW * m);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int d = wv[j][c];
+        const float wf[4] = {sbyte_f32<0>(d) * sc[0][j], sbyte_f32<1>(d) * sc[0][j], sbyte_f32<2>(d) * sc[0][j],
+                             sbyte_f32<3>(d) * sc[0][j]};
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          f32x4 t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) t = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[q], x[m][q], t, 0, 0, 0);
+          if (c % 2 == 0) part[c / 2][j][m] = t;
+          else part[c / 2][j][m] += t;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[0][j][m] += part[0][j][m] + part[1][j][m];
+  };
+  auto mul = [&](i32x4 (&w)[P][NT], int i, int st) {
+    if constexpr (F32) mul32(w, i, st);
+    else mul16(w, i, st);
   };
 
   // Group i: the activation copies, then the weights, of iteration i.  D groups are in
@@ -291,14 +344,23 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
     for (int t = 0; t < MT; ++t) {
       const int m = bm + 16 * t + col;
       if (m >= p.M) continue;
-      if (p.S == 1) {
+      if (p.S == 1 && F32) {
+        float* yr = static_cast<float*>(L0.y) + (int64_t)m * L0.ldy + nb;
+        if (full) {
+          *reinterpret_cast<f32x4*>(yr) = sum[0][j][t];
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (nb + q < N) yr[q] = sum[0][j][t][q];
+        }
+      } else if (p.S == 1) {
         uint16_t o[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           float v[P];
 #pragma unroll
           for (int pl = 0; pl < P; ++pl) v[pl] = sum[pl][j][t][q];
-          o[q] = w8a16_out<P, F16>(v);
+          o[q] = w8a16_out<P, XT == QS_F16>(v);
         }
         uint16_t* yr = static_cast<uint16_t*>(L0.y) + (int64_t)m * L0.ldy + nb;
         if (full) {
@@ -327,7 +389,7 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
 
 // Slice sums in slice order and the epilogue: one thread per (row m, 4 columns of the
 // partial row); every linear's N is a multiple of 4 (the host checks).
-template <int P, bool F16>
+template <int P, int XT>
 __global__ __launch_bounds__(256) void k_prefill_reduce(PfParams p) {
   const int q4 = p.n_total / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -349,13 +411,23 @@ __global__ __launch_bounds__(256) void k_prefill_reduce(PfParams p) {
     for (int s = 1; s < p.S; ++s) a[pl] += *reinterpret_cast<const f32x4*>(pr + s * step);
   }
   const PfLin& L = p.lin[li];
+  if constexpr (XT == QS_F32) {
+    float* yr = static_cast<float*>(L.y) + (int64_t)m * L.ldy + (ncol - L.n_begin);
+    if (p.vec) {
+      *reinterpret_cast<f32x4*>(yr) = a[0];
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) yr[q] = a[0][q];
+    }
+    return;
+  }
   uint16_t o[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     float v[P];
 #pragma unroll
     for (int pl = 0; pl < P; ++pl) v[pl] = a[pl][q];
-    o[q] = w8a16_out<P, F16>(v);
+    o[q] = w8a16_out<P, XT == QS_F16>(v);
   }
   uint16_t* yr = static_cast<uint16_t*>(L.y) + (int64_t)m * L.ldy + (ncol - L.n_begin);
   if (p.vec) {
@@ -366,11 +438,12 @@ __global__ __launch_bounds__(256) void k_prefill_reduce(PfParams p) {
   }
 }
 
-// Tile shapes: MT, NT * P, WN, WK, and three times in microseconds fitted to 600 timings of
-// these shapes (M 33..1531; 2048x1536, 1536x8960, 6144x4096, 4096x14336 and 1024x2816 plain,
-// 8960x1536, 14336x4096 and 2816x1024 paired; 8% rms): `lat` a round of WK 64-k steps of one
-// workgroup alone on a CU, `thr` the same per workgroup when a CU has several, `end` its
-// start and epilogue per workgroup.
+// Tile shapes: MT, NT * P, WN, WK, and three times in microseconds fitted to timings of these
+// shapes: `lat` a round of WK 64-k steps of one workgroup alone on a CU, `thr` the same per
+// workgroup when a CU has several, `end` its start and epilogue per workgroup.  16-bit: 600
+// timings (M 33..1531; 2048x1536, 1536x8960, 6144x4096, 4096x14336 and 1024x2816 plain,
+// 8960x1536, 14336x4096 and 2816x1024 paired; 8% rms).  fp32: 600 timings (M 2..500;
+// 1536x8960, 4096x1024, 8960x1536, 2500x320, 3000x1536, 4096x4096, 4096x14336; 6% rms).
 struct PfShape {
   int MT, NTP, WN, WK;
   float lat, thr, end;
@@ -378,7 +451,9 @@ struct PfShape {
 constexpr PfShape kPfShapes[] = {
     {2, 2, 4, 2, 0.14f, 0.59f, 0.47f}, {4, 2, 4, 2, 0.73f, 0.65f, 0.70f},
     {8, 2, 4, 1, 0.61f, 0.48f, 0.36f}, {8, 2, 4, 2, 0.32f, 0.90f, 2.81f},
+    {1, 1, 4, 2, 0.91f, 0.75f, 0.30f}, {2, 1, 4, 2, 1.42f, 1.27f, 0.93f},  // fp32
 };
+constexpr int kPfShapes16 = 4, kPfShapesAll = 6;
 constexpr float kPfLaunch = 4.1f;         // a launch
 constexpr float kPfReduce = 2.7f;         // the reduce launch,
 constexpr float kPfReduceBytes = 4.8e6f;  // and its partial bytes (written and read) per microsecond
@@ -392,9 +467,9 @@ struct PfPlan {
 
 // The shape and slice count with the smallest modelled time: a large tile reuses its operands
 // best, a small one (or a K split, which costs a reduce launch) fills the chip when the
-// product has few tiles.  Over the 70 products timed for the fit, the choice is 2% slower than
-// the best of seven shapes on average and 21% at worst (33..64 rows of 14336x4096 paired).
-PfPlan pf_plan(int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool split) {
+// product has few tiles.  Over the products timed for the fits, the choice is 2% (16-bit) and
+// 3% (fp32) slower than the best shape on average and 21% at worst.
+PfPlan pf_plan(bool f32, int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool split) {
   const int64_t T = K / 64;
   int64_t n_total = 0;
   for (int i = 0; i < (P == 2 ? 1 : n_lin); ++i) {
@@ -403,7 +478,7 @@ PfPlan pf_plan(int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool sp
   }
   PfPlan best{0, 1, 0, n_total};
   float best_t = 0.f;
-  for (int k = 0; k < (int)(sizeof(kPfShapes) / sizeof(kPfShapes[0])); ++k) {
+  for (int k = f32 ? kPfShapes16 : 0; k < (f32 ? kPfShapesAll : kPfShapes16); ++k) {
     const PfShape& sh = kPfShapes[k];
     int64_t tiles_n = 0;
     for (int i = 0; i < (P == 2 ? 1 : n_lin); ++i) tiles_n += cdiv(N[i], 16 * sh.NTP / P * sh.WN);
@@ -425,40 +500,46 @@ PfPlan pf_plan(int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool sp
   return best;
 }
 
-template <int P, bool F16>
+template <int P, int XT>
 void pf_launch(const PfParams& p, int shape, hipStream_t s) {
   const dim3 grid((unsigned)((int64_t)p.tiles_m * p.tiles_n * p.S));
-#define QS_PF(K_)                                                                                                 \
-  if (shape == K_) {                                                                                              \
-    constexpr PfShape h = kPfShapes[K_];                                                                          \
-    hipLaunchKernelGGL((k_prefill<P, h.MT, h.NTP / P, h.WN, h.WK, 2, F16>), grid, dim3(h.WN * h.WK * 64), 0, s, p); \
+#define QS_PF(K_)                                                                                               \
+  if (shape == K_) {                                                                                            \
+    constexpr PfShape h = kPfShapes[K_];                                                                        \
+    hipLaunchKernelGGL((k_prefill<P, h.MT, h.NTP / P, h.WN, h.WK, 2, XT>), grid, dim3(h.WN * h.WK * 64), 0, s, p); \
   }
-  QS_PF(0) QS_PF(1) QS_PF(2) QS_PF(3)
+  if constexpr (XT == QS_F32) {
+    QS_PF(4) QS_PF(5)
+  } else {
+    QS_PF(0) QS_PF(1) QS_PF(2) QS_PF(3)
+  }
 #undef QS_PF
   if (p.S > 1) {
     const dim3 rg((unsigned)cdiv((int64_t)p.M * (p.n_total / 4), 256));
-    hipLaunchKernelGGL((k_prefill_reduce<P, F16>), rg, dim3(256), 0, s, p);
+    hipLaunchKernelGGL((k_prefill_reduce<P, XT>), rg, dim3(256), 0, s, p);
   }
 }
 
 }  // namespace
 
-// W8A16 over the linears' shared x: `lin` holds the P planes of a SwiGLU (P = 2, y in lin[0])
+// y = x @ W^T over the linears' shared x: `lin` holds the P planes of a SwiGLU (P = 2, y in lin[0])
 // or n_lin linears.  `workspace` null: no K split.  Returns QS_ERR_UNSUPPORTED, without a
 // message, for operands the kernel does not take (the callers' other kernels do).
-int run_prefill(const void* x, bool f16, int64_t ldx, int n_lin, const QrowPrefillLin* lin, int P, int64_t M,
+int run_prefill(const void* x, int x_dtype, int64_t ldx, int n_lin, const QrowPrefillLin* lin, int P, int64_t M,
                 int64_t K, void* workspace, size_t workspace_bytes, hipStream_t s) {
-  if (K % 64 != 0 || ldx % 8 != 0 || !aligned(x, 16)) return QS_ERR_UNSUPPORTED;
-  if (128 * ldx * 2 >= INT_MAX || 128 * K >= INT_MAX) return QS_ERR_UNSUPPORTED;  // tile offsets are 31-bit
+  const bool f32 = x_dtype == QS_F32;
+  const int es = f32 ? 4 : 2;
+  if (K % 64 != 0 || ldx * es % 16 != 0 || !aligned(x, 16)) return QS_ERR_UNSUPPORTED;
+  if (128 * ldx * 4 >= INT_MAX || 128 * K >= INT_MAX) return QS_ERR_UNSUPPORTED;  // tile offsets are 31-bit
   PfParams p{};
   int64_t N[4];
   bool vec = true;
   for (int i = 0; i < n_lin; ++i) {
     if (!aligned(lin[i].codes, 16)) return QS_ERR_UNSUPPORTED;
     N[i] = lin[i].N;
-    if (lin[i].y) vec = vec && lin[i].ldy % 4 == 0 && aligned(lin[i].y, 8);
+    if (lin[i].y) vec = vec && lin[i].ldy % 4 == 0 && aligned(lin[i].y, 4 * es);
   }
-  const PfPlan plan = pf_plan(M, n_lin, N, K, P, workspace != nullptr);
+  const PfPlan plan = pf_plan(f32, M, n_lin, N, K, P, workspace != nullptr);
   const PfShape& sh = kPfShapes[plan.shape];
   if (plan.S > 1) {
     if (workspace_bytes < (size_t)plan.S * P * M * plan.n_total * 4)
@@ -467,7 +548,7 @@ int run_prefill(const void* x, bool f16, int64_t ldx, int n_lin, const QrowPrefi
   }
   const int64_t tiles_m = cdiv(M, 16 * sh.MT);
   if (tiles_m * plan.tiles_n * plan.S > INT_MAX || plan.n_total > INT_MAX) return QS_ERR_UNSUPPORTED;
-  p.x = static_cast<const uint16_t*>(x);
+  p.x = x;
   p.ldx = ldx;
   p.M = (int)M;
   p.K = (int)K;
@@ -488,9 +569,10 @@ int run_prefill(const void* x, bool f16, int64_t ldx, int n_lin, const QrowPrefi
       nb += N[i];
     }
   }
-  if (P == 2) pf_launch<2, false>(p, plan.shape, s);
-  else if (f16) pf_launch<1, true>(p, plan.shape, s);
-  else pf_launch<1, false>(p, plan.shape, s);
+  if (P == 2) pf_launch<2, QS_BF16>(p, plan.shape, s);
+  else if (f32) pf_launch<1, QS_F32>(p, plan.shape, s);
+  else if (x_dtype == QS_F16) pf_launch<1, QS_F16>(p, plan.shape, s);
+  else pf_launch<1, QS_BF16>(p, plan.shape, s);
   return hip_check(hipGetLastError(), "k_prefill launch");
 }
 
@@ -498,10 +580,11 @@ int run_prefill(const void* x, bool f16, int64_t ldx, int n_lin, const QrowPrefi
 
 using namespace qs;
 
-extern "C" size_t qs_qrow_prefill_workspace_bytes(int64_t M, int n_linear, const int64_t* N, int64_t K, int swiglu) {
+extern "C" size_t qs_qrow_prefill_workspace_bytes(int x_dtype, int64_t M, int n_linear, const int64_t* N, int64_t K,
+                                                  int swiglu) {
   if (!N || n_linear < 1 || n_linear > 4 || M < 1 || K < 64) return 0;
   const int P = swiglu ? 2 : 1;
-  const PfPlan plan = pf_plan(M, n_linear, N, K, P, true);
+  const PfPlan plan = pf_plan(x_dtype == QS_F32, M, n_linear, N, K, P, true);
   return plan.S > 1 ? (size_t)plan.S * P * M * plan.n_total * 4 : 0;
 }
 
@@ -509,7 +592,8 @@ namespace {
 
 int prefill_check(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K) {
   if (!x) return fail(QS_ERR_INVALID, "qrow prefill: null activations");
-  if (x_dtype != QS_BF16 && x_dtype != QS_F16) return fail(QS_ERR_INVALID, "qrow prefill: activations BF16 or F16");
+  if (x_dtype != QS_BF16 && x_dtype != QS_F16 && x_dtype != QS_F32)
+    return fail(QS_ERR_INVALID, "qrow prefill: activations BF16, F16 or F32");
   if (M < 1 || K < 1 || ldx < K) return fail(QS_ERR_INVALID, "qrow prefill: bad M, K or ldx");
   if (M > (int64_t)1 << 30 || K > (int64_t)1 << 30) return fail(QS_ERR_LIMIT, "qrow prefill: dimension exceeds 2^30");
   return QS_OK;
@@ -537,7 +621,7 @@ extern "C" int qs_qrow_matmul_prefill(const void* x, int x_dtype, int64_t ldx, i
       return fail(QS_ERR_INVALID, "qrow prefill: bad N/ldy for linear %d", i);
     lin[i] = QrowPrefillLin{codes[i], scales[i], y[i], ldy[i], N[i]};
   }
-  return prefill_status(run_prefill(x, x_dtype == QS_F16, ldx, n_linear, lin, 1, M, K,
+  return prefill_status(run_prefill(x, x_dtype, ldx, n_linear, lin, 1, M, K,
                                     workspace_bytes ? workspace : nullptr, workspace_bytes,
                                     static_cast<hipStream_t>(stream)));
 }
@@ -551,6 +635,6 @@ extern "C" int qs_qrow_swiglu_prefill(const void* x, int64_t ldx, const int8_t* 
     return fail(QS_ERR_INVALID, "swiglu prefill: null pointer");
   if (N <= 0 || N > ((int64_t)1 << 30) || ldy < N) return fail(QS_ERR_INVALID, "swiglu prefill: bad N/ldy");
   const QrowPrefillLin lin[2] = {{gate_codes, gate_scales, y, ldy, N}, {up_codes, up_scales, nullptr, 0, N}};
-  return prefill_status(run_prefill(x, false, ldx, 2, lin, 2, M, K, workspace_bytes ? workspace : nullptr,
+  return prefill_status(run_prefill(x, QS_BF16, ldx, 2, lin, 2, M, K, workspace_bytes ? workspace : nullptr,
                                     workspace_bytes, static_cast<hipStream_t>(stream)));
 }

@@ -1768,20 +1768,32 @@ void launch_top2_mb(const QrowParams& q, int rows, int start_row, float* pv, int
 // blocks; the fused path uses 8-row blocks, so this bounds both).
 int64_t top2_blocks(int64_t rows) { return cdiv(rows, 4); }
 
+// Whether a call takes the prefill kernel: 16-bit rows past a 32-row batch; fp32 rows that
+// would need three VALU launches, or two for three or more rows (4096 x 1024: three rows
+// 8.4 -> 8.1 us, two 7.1 against 8.1; 1536 x 8960: three rows 17.8 -> 15.5, two 11.7 against
+// 15.6).  Single rows always keep the decode kernels.
+bool many_rows(const QrowParams& p, int x_dtype, int64_t M) {
+  if (x_dtype != QS_F32) return M > 32;
+  if (M < 2) return false;
+  if (!valu_eligible(p, x_dtype)) return true;
+  const int64_t launches = cdiv(M, valu_mb(x_dtype, p.K, M));
+  return launches >= 3 || (launches == 2 && M >= 3);
+}
+
 // Runs one set of linears sharing x.
 int run_linears(QrowParams p, int x_dtype, int64_t M, hipStream_t s, bool row_stable) {
   if (M == 0) return QS_OK;
   const int esz = x_dtype == QS_F32 ? 4 : 2;
-  // decode-sized batches (and the row-stable contract) take the VALU path
-  if ((row_stable || M <= kValuRows || x_dtype == QS_F32) && valu_eligible(p, x_dtype))
-    return run_valu(p, x_dtype, M, s, false);
-  if (!row_stable && M > 32 && x_dtype != QS_F32) {  // one launch for all rows (qs_prefill.hip)
+  if (!row_stable && many_rows(p, x_dtype, M)) {  // one launch for all rows (qs_prefill.hip)
     QrowPrefillLin lin[4];
     for (int i = 0; i < p.n_lin; ++i)
       lin[i] = QrowPrefillLin{p.lin[i].codes, p.lin[i].scales, p.lin[i].y, p.lin[i].ldy, p.lin[i].N};
-    const int st = run_prefill(p.x, x_dtype == QS_F16, p.ldx, p.n_lin, lin, 1, M, p.K, nullptr, 0, s);
+    const int st = run_prefill(p.x, x_dtype, p.ldx, p.n_lin, lin, 1, M, p.K, nullptr, 0, s);
     if (st != QS_ERR_UNSUPPORTED) return st;
   }
+  // decode-sized batches (and the row-stable contract) take the VALU path
+  if ((row_stable || M <= kValuRows || x_dtype == QS_F32) && valu_eligible(p, x_dtype))
+    return run_valu(p, x_dtype, M, s, false);
   if (!row_stable && mfma_eligible(p, x_dtype)) {
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
       QrowParams q = p;
@@ -1944,7 +1956,7 @@ extern "C" int qs_qrow_swiglu(const void* x, int64_t ldx, const int8_t* gate_cod
   if (M <= kValuRows && valu_eligible(p, QS_BF16)) return run_valu(p, QS_BF16, M, s, true);
   if (M > 32) {
     const QrowPrefillLin lin[2] = {{gate_codes, gate_scales, y, ldy, N}, {up_codes, up_scales, nullptr, 0, N}};
-    st = run_prefill(x, false, ldx, 2, lin, 2, M, K, nullptr, 0, s);
+    st = run_prefill(x, QS_BF16, ldx, 2, lin, 2, M, K, nullptr, 0, s);
     if (st != QS_ERR_UNSUPPORTED) return st;
   }
   if (mfma_eligible(p, QS_BF16)) {

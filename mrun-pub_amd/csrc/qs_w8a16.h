@@ -1,4 +1,4 @@
-// Pieces shared by the W8A16 MFMA kernels (qs_batched.hip, qs_prefill.hip).
+// Pieces shared by the MFMA qrow kernels (qs_batched.hip, qs_prefill.hip).
 #pragma once
 
 #include "qs_common.h"
@@ -41,7 +41,7 @@ __device__ __forceinline__ uint16_t w8a16_out(const float (&v)[P]) {
   }
 }
 
-// One linear of a W8A16 call with many activation rows (qs_prefill.hip).
+// One linear of a call with many activation rows (qs_prefill.hip).
 struct QrowPrefillLin {
   const int8_t* codes;
   const float* scales;
@@ -49,7 +49,7 @@ struct QrowPrefillLin {
   int64_t ldy;
   int64_t N;
 };
-int run_prefill(const void* x, bool f16, int64_t ldx, int n_lin, const QrowPrefillLin* lin, int P, int64_t M,
+int run_prefill(const void* x, int x_dtype, int64_t ldx, int n_lin, const QrowPrefillLin* lin, int P, int64_t M,
                 int64_t K, void* workspace, size_t workspace_bytes, hipStream_t s);
 
 }  // namespace qs

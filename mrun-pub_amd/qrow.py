@@ -169,39 +169,29 @@ def _batched_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool 
             and x2.stride(0) == k and x2.data_ptr() % 16 == 0 and all(c.data_ptr() % 16 == 0 for c in codes))
 
 
+def _many_f32_rows(m: int, k: int) -> bool:
+    """fp32 rows that take the prefill kernel: those that would need three launches of the VALU
+    kernel (which stages 4, 2 or 1 rows of k floats in 64 KiB of LDS; none past k = 12288), or
+    two for three or more rows.  The C entry points' rule, with its timings, is many_rows()."""
+    if m < 2 or k > 12288:
+        return m >= 2
+    mb = next((b for b in (4, 2) if b * k * 4 <= 65536 and b <= m), 1)
+    launches = -(-m // mb)
+    return launches >= 3 or (launches == 2 and m >= 3)
+
+
 def _prefill_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool = False) -> bool:
-    """More rows than a batch, in the layout qs_qrow_matmul_prefill takes (rows of whole 64-k
-    steps, 16-byte aligned; the offsets inside a 128-row tile are 31-bit)."""
+    """More rows than the decode and batched kernels take, in the layout qs_qrow_matmul_prefill
+    does (rows of whole 64-k steps, 16-byte aligned; offsets inside a 128-row tile are 31-bit)."""
     m, k = int(x2.shape[0]), int(x2.shape[1])
-    return (m > BATCHED_MAX_M and x2.dtype in (torch.bfloat16, torch.float16)
-            and (not swiglu or x2.dtype == torch.bfloat16) and k % 64 == 0 and k < 1 << 22
+    many = _many_f32_rows(m, k) if x2.dtype == torch.float32 else m > BATCHED_MAX_M
+    return (many and (not swiglu or x2.dtype == torch.bfloat16) and k % 64 == 0 and k < 1 << 22
             and x2.stride(0) == k and x2.data_ptr() % 16 == 0 and all(c.data_ptr() % 16 == 0 for c in codes))
-
-
-def _run_many(kind: str, x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
-              swiglu: bool) -> None:
-    """``qs_qrow_matmul_<kind>`` / ``qs_qrow_swiglu_<kind>`` (kind: batched or prefill) with a
-    workspace for the K-slice partial sums."""
-    device = x2.device
-    m, k = int(x2.shape[0]), int(x2.shape[1])
-    ns = [int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]]
-    stream = nat.stream_of(device)
-    n_arr = nat.int64_array(ns)
-    ws_bytes = int(getattr(nat.load(), f"qs_qrow_{kind}_workspace_bytes")(m, len(ns), n_arr, k, int(swiglu)))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=device)
-    if swiglu:
-        (gc, gs), (uc, us) = pages
-        nat.call(f"qs_qrow_swiglu_{kind}", nat.ptr(x2), k, nat.ptr(gc), nat.ptr(gs), nat.ptr(uc), nat.ptr(us),
-                 nat.ptr(outs[0]), ns[0], m, ns[0], k, nat.ptr(ws), ws_bytes, stream)
-    else:
-        nat.call(f"qs_qrow_matmul_{kind}", nat.ptr(x2), nat.dtype_code(x2.dtype), k, len(pages),
-                 nat.pointer_array([nat.ptr(c) for c, _ in pages]), nat.pointer_array([nat.ptr(sc) for _, sc in pages]),
-                 nat.pointer_array([nat.ptr(o) for o in outs]), n_arr, n_arr, m, k, nat.ptr(ws), ws_bytes, stream)
 
 
 def _run_batched(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
                  swiglu: bool) -> None:
-    """At most 32 rows through the batched kernels (the split depends on N and K only)."""
+    """At most 32 16-bit rows through the batched kernels (the split depends on N and K only)."""
     _run_many("batched", x2, pages, outs, swiglu)
 
 
@@ -209,6 +199,31 @@ def _run_prefill(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]
                  swiglu: bool) -> None:
     """Any number of rows through the prefill kernel."""
     _run_many("prefill", x2, pages, outs, swiglu)
+
+
+def _run_many(kind: str, x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
+              swiglu: bool) -> None:
+    """``qs_qrow_matmul_<kind>`` / ``qs_qrow_swiglu_<kind>`` with a workspace for the K-slice
+    partial sums."""
+    device = x2.device
+    m, k = int(x2.shape[0]), int(x2.shape[1])
+    ns = [int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]]
+    stream = nat.stream_of(device)
+    n_arr = nat.int64_array(ns)
+    lib, xdt = nat.load(), nat.dtype_code(x2.dtype)
+    if kind == "batched":
+        ws_bytes = int(lib.qs_qrow_batched_workspace_bytes(m, len(ns), n_arr, k, int(swiglu)))
+    else:
+        ws_bytes = int(lib.qs_qrow_prefill_workspace_bytes(xdt, m, len(ns), n_arr, k, int(swiglu)))
+    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=device)
+    if swiglu:
+        (gc, gs), (uc, us) = pages
+        nat.call(f"qs_qrow_swiglu_{kind}", nat.ptr(x2), k, nat.ptr(gc), nat.ptr(gs), nat.ptr(uc), nat.ptr(us),
+                 nat.ptr(outs[0]), ns[0], m, ns[0], k, nat.ptr(ws), ws_bytes, stream)
+    else:
+        nat.call(f"qs_qrow_matmul_{kind}", nat.ptr(x2), xdt, k, len(pages),
+                 nat.pointer_array([nat.ptr(c) for c, _ in pages]), nat.pointer_array([nat.ptr(sc) for _, sc in pages]),
+                 nat.pointer_array([nat.ptr(o) for o in outs]), n_arr, n_arr, m, k, nat.ptr(ws), ws_bytes, stream)
 
 
 @torch.inference_mode()
@@ -236,9 +251,9 @@ def qrow_matmul(
         flat = flat.contiguous()
     m = int(flat.shape[0])
     y = _out_buffer(out, m, n, x.dtype, device)
-    if m and not row_stable and _batched_eligible(flat, [codes]):
+    if m > 1 and not row_stable and _batched_eligible(flat, [codes]):
         _run_batched(flat, [(codes, scales)], [y], swiglu=False)
-    elif m and not row_stable and _prefill_eligible(flat, [codes]):
+    elif m > 1 and not row_stable and _prefill_eligible(flat, [codes]):
         _run_prefill(flat, [(codes, scales)], [y], swiglu=False)
     elif m:
         nat.call(
@@ -279,9 +294,9 @@ def qrow_matmul_multi(
     if out is not None and len(out) != len(pages):
         raise ValueError("one output buffer per linear")
     outs = [_out_buffer(None if out is None else out[i], m, n, x.dtype, device) for i, (n, _) in enumerate(shapes)]
-    if m and _batched_eligible(flat, [c for c, _ in pages]):
+    if m > 1 and _batched_eligible(flat, [c for c, _ in pages]):
         _run_batched(flat, pages, outs, swiglu=False)
-    elif m and _prefill_eligible(flat, [c for c, _ in pages]):
+    elif m > 1 and _prefill_eligible(flat, [c for c, _ in pages]):
         _run_prefill(flat, pages, outs, swiglu=False)
     elif m:
         nat.call(
@@ -378,9 +393,9 @@ def qrow_swiglu_into(gate_page: CompactQRowPage, up_page: CompactQRowPage, activ
     flat = activations.reshape(-1, k).contiguous()
     m = int(flat.shape[0])
     y = _out_buffer(out, m, n, torch.bfloat16, device)
-    if m and _batched_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
+    if m > 1 and _batched_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
         _run_batched(flat, [(gate_page.codes, gate_page.scales), (up_page.codes, up_page.scales)], [y], swiglu=True)
-    elif m and _prefill_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
+    elif m > 1 and _prefill_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
         _run_prefill(flat, [(gate_page.codes, gate_page.scales), (up_page.codes, up_page.scales)], [y], swiglu=True)
     elif m:
         nat.call(

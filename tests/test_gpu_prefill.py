@@ -118,3 +118,58 @@ def test_prefill_nonfinite_stays_in_its_row(dev):
     rows = np.array([r for r in range(m) if r not in (5, 69)])
     assert np.isfinite(y[rows]).all() and not np.isfinite(y[5]).any() and np.isnan(y[69]).all()
     assert oq.rel_l2(y[rows], oq.qrow_matmul_w8a16(codes, scales, x[rows])) <= TOL
+
+
+# fp32: 16 / 32-row tiles, 64-row weight blocks, ragged N, short and split K.  Both sides sum
+# exact products of the same fp32 weights in some order; the longest chains here are 16
+# products, then about sqrt(K) partial sums, so a result lies within 2 (16 + sqrt(K)) 2^-24 of
+# the norm of its terms, 3e-7 of rel-L2 on random signs (1e-5 is the fp32 contract).
+@pytest.mark.parametrize("m", [5, 16, 17, 33, 149])
+@pytest.mark.parametrize("n,k", [(5, 64), (63, 128), (65, 320), (300, 1536), (72, 8960), (1030, 1088)])
+def test_prefill_fp32(dev, m, n, k):
+    from mrun_pub_amd import qrow as q
+
+    codes, scales = _case(n, k, seed=m + n + k)
+    x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+    c, s, xd = (torch.from_numpy(a).to(dev) for a in (codes, scales, x))
+    assert q._prefill_eligible(xd, [c])
+    ref = x.astype(np.float64) @ oq.dequant_qrow(codes, scales).astype(np.float64).T
+    buf, out = _guarded(m, n, torch.float32, dev)
+    q.qrow_matmul(c, s, xd, out=out)
+    assert oq.rel_l2(out.cpu().numpy(), ref) <= 1e-6
+    assert _untouched(buf, m, n)
+    buf, out = _guarded(m, n, torch.float32, dev)
+    q.nat.call("qs_qrow_matmul", xd.data_ptr(), q.nat.QS_F32, k, c.data_ptr(), s.data_ptr(), out.data_ptr(), n, m, n, k,
+               q.nat.stream_of(dev))
+    assert oq.rel_l2(out.cpu().numpy(), ref) <= 1e-6
+    assert _untouched(buf, m, n)
+
+
+def test_prefill_fp32_long_rows_and_range(dev):
+    """Rows past the decode kernel's 12288 k, values near both ends of fp32, and a non-finite
+    activation that reaches its own row only."""
+    from mrun_pub_amd import qrow as q
+
+    n, k, m = 40, 14336, 6
+    codes, scales = _case(n, k, seed=9)
+    x = np.random.default_rng(10).standard_normal((m, k)).astype(np.float32)
+    x[1] *= np.float32(1e-38)  # subnormal activations among them
+    x[2] *= np.float32(2e33)
+    x[3, 7] = np.inf
+    c, s, xd = (torch.from_numpy(a).to(dev) for a in (codes, scales, x))
+    assert q._prefill_eligible(xd, [c])
+    y = q.qrow_matmul(c, s, xd).cpu().numpy()
+    ref = x.astype(np.float64) @ oq.dequant_qrow(codes, scales).astype(np.float64).T
+    for r in (0, 1, 2, 4, 5):
+        assert oq.rel_l2(y[r], ref[r]) <= 1e-6, r
+    assert not np.isfinite(y[3]).any()
+
+
+def test_many_f32_rows_rule(dev):
+    """Which fp32 row counts leave the decode kernel: the Python rule equals the C one."""
+    from mrun_pub_amd import qrow as q
+
+    assert [m for m in range(1, 9) if not q._many_f32_rows(m, 1024)] == [1, 2, 4]
+    assert [m for m in range(1, 9) if not q._many_f32_rows(m, 8192)] == [1, 2]
+    assert [m for m in range(1, 9) if not q._many_f32_rows(m, 12288)] == [1, 2]
+    assert [m for m in range(1, 9) if not q._many_f32_rows(m, 16384)] == [1]
