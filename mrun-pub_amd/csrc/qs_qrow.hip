@@ -1277,6 +1277,141 @@ __global__ __launch_bounds__(512) void k_gemv_top2_xg(QrowParams p, int rows, in
   block_top2<WPB, MB>(v1, i1, v2, i2, p.M, part_v, part_i);
 }
 
+// The same search for 3 to 16 activation rows on the matrix pipe.  The head is a weight
+// stream: k_gemv_top2_xg's register activations hold at most two rows, so eleven rows of a
+// 151,665 x 1536 head read it six times (6 x 50 us); here it is read once.  The rows' 16-row
+// MFMA tile sits in LDS once per workgroup (16-byte chunk j of row m at slot j ^ m, so a
+// fragment read's 16 rows fall in distinct bank groups), and each wave walks 16-row weight
+// tiles on its own, no barriers, with W 64-k chunks (16 rows x 64 bytes a load) in flight
+// across tile boundaries.  Dequantized weights are the A operand, so lane l holds the logits
+// of weight rows 4 (l >> 4) + 0..3 for activation row l & 15 and keeps that row's running
+// first and second.  Four accumulators per tile keep the fp32 chains as short as the VALU
+// kernel's.  Eleven bf16 rows: 269 -> 67 us with the rerank (this
+// launch 55); fp32 rows run 16x16x4 MFMAs,
+// whose rate bounds them (eleven rows of
+// 151,936 x 1536 without the rerank: 315 -> 117 us; bf16 292 -> 61).
+template <int XT, int W>
+__global__ __launch_bounds__(512) void k_head_top2(QrowParams p, int rows, int start_row, float* part_v,
+                                                   int* part_i) {
+  constexpr bool F32 = XT == QS_F32;
+  constexpr int ES = F32 ? 4 : 2, WPB = 8;
+  typedef Half<XT == QS_F16> H;
+  typedef typename H::vec hvec;
+  extern __shared__ __attribute__((aligned(16))) uint8_t xs[];  // [16][K * ES]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, grp = lane >> 4;
+  const int K = p.K, C = K / 64, RB = K * ES, RC = RB / 16;
+  const int ntiles = (rows + 15) / 16, stride = (int)gridDim.x * WPB;
+  const int8_t* codes = p.lin[0].codes;
+  const float* scales = p.lin[0].scales;
+
+  // load position: chunk lc of tile lt (the last tile is read again past the end)
+  int lt = (int)blockIdx.x * WPB + wave, lc = 0;
+  const int8_t* lp;
+  float scn;
+  auto enter = [&]() {
+    const int n = 16 * lt + col;
+    const int r = n < rows ? n : rows - 1;
+    lp = codes + (int64_t)r * K + 16 * grp;
+    scn = scales[r];
+  };
+  enter();
+  i32x4 w[W];
+  auto load = [&](i32x4& dst) {
+    if (lc == C) {
+      lc = 0;
+      lt += stride;
+      enter();
+    }
+    dst = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(lp + 64 * lc));
+    ++lc;
+  };
+#pragma unroll
+  for (int u = 0; u < W; ++u) load(w[u]);
+
+  for (int e = tid; e < 16 * RC; e += 512) {
+    const int m = e / RC, j = e - m * RC;
+    i32x4 v{0, 0, 0, 0};
+    if (m < p.M) v = *reinterpret_cast<const i32x4*>(static_cast<const uint8_t*>(p.x) + (int64_t)m * p.ldx * ES + 16 * j);
+    *reinterpret_cast<i32x4*>(xs + m * RB + 16 * (j ^ m)) = v;
+  }
+  __syncthreads();
+
+  float v1 = -INFINITY, v2 = -INFINITY;
+  int i1 = INT_MAX, i2 = INT_MAX;
+  const uint8_t* xrow = xs + col * RB;
+  for (int ct = (int)blockIdx.x * WPB + wave; ct < ntiles; ct += stride) {
+    const float sc = scn;  // the load position is still inside this tile: W <= C
+    f32x4 acc[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < C; c0 += W) {
+#pragma unroll
+      for (int u = 0; u < W; ++u) {
+        const int c = c0 + u;
+        const i32x4 d = w[u];
+        load(w[u]);
+        if constexpr (F32) {
+          f32x4 t[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(xrow + 16 * ((16 * c + 4 * grp + j) ^ col));
+            const float wf[4] = {sbyte_f32<0>(d[j]) * sc, sbyte_f32<1>(d[j]) * sc, sbyte_f32<2>(d[j]) * sc,
+                                 sbyte_f32<3>(d[j]) * sc};
+            t[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) t[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[q], x[q], t[j], 0, 0, 0);
+          }
+          acc[u & 3] += (t[0] + t[1]) + (t[2] + t[3]);
+        } else {
+          hvec b0, b1;
+          H::deq(d, sc, b0, b1);
+          const hvec x0 = *reinterpret_cast<const hvec*>(xrow + 16 * ((8 * c + 2 * grp) ^ col));
+          const hvec x1 = *reinterpret_cast<const hvec*>(xrow + 16 * ((8 * c + 2 * grp + 1) ^ col));
+          acc[2 * (u & 1)] = H::mma(b0, x0, acc[2 * (u & 1)]);
+          acc[2 * (u & 1) + 1] = H::mma(b1, x1, acc[2 * (u & 1) + 1]);
+        }
+      }
+    }
+    const f32x4 v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = 16 * ct + 4 * grp + q;
+      if (n < rows) top2_push(v[q], start_row + n, v1, i1, v2, i2);
+    }
+  }
+  // the four lane groups hold different rows of the same activation row
+#pragma unroll
+  for (int off = 16; off <= 32; off <<= 1) {
+    const float o1 = __shfl_xor(v1, off), o2 = __shfl_xor(v2, off);
+    const int j1 = __shfl_xor(i1, off), j2 = __shfl_xor(i2, off);
+    top2_push(o1, j1, v1, i1, v2, i2);
+    top2_push(o2, j2, v1, i1, v2, i2);
+  }
+  __syncthreads();  // the activations are no longer read
+  float* tv = reinterpret_cast<float*>(xs);  // [WPB][16][2]
+  int* ti = reinterpret_cast<int*>(tv + WPB * 32);
+  if (lane < 16) {
+    tv[(wave * 16 + lane) * 2] = v1;
+    ti[(wave * 16 + lane) * 2] = i1;
+    tv[(wave * 16 + lane) * 2 + 1] = v2;
+    ti[(wave * 16 + lane) * 2 + 1] = i2;
+  }
+  __syncthreads();
+  if (tid < p.M) {
+    float a1 = -INFINITY, a2 = -INFINITY;
+    int b1 = INT_MAX, b2 = INT_MAX;
+    for (int e = 0; e < WPB; ++e)
+      for (int h = 0; h < 2; ++h) top2_push(tv[(e * 16 + tid) * 2 + h], ti[(e * 16 + tid) * 2 + h], a1, b1, a2, b2);
+    const int64_t o = ((int64_t)tid * gridDim.x + blockIdx.x) * 2;
+    part_v[o] = a1;
+    part_i[o] = b1;
+    part_v[o + 1] = a2;
+    part_i[o + 1] = b2;
+  }
+}
+
 // Any K / alignment: one wave per row, one activation row per launch (x points at it),
 // the same arithmetic contract as k_generic.
 __global__ __launch_bounds__(256) void k_generic_top2(QrowParams p, int x_dtype, int rows, int start_row,
@@ -2009,6 +2144,31 @@ int top2_validate(const void* x, int x_dtype, int64_t ldx, const int8_t* codes, 
   return QS_OK;
 }
 
+// k_head_top2: three or more 16-bit rows (two still fit the register kernel; 151,936 x 1536:
+// two rows 48 us, three 106 -> 59), five or more fp32 rows (four are one VALU launch, 124 us),
+// whose 16-row tile fits LDS.
+bool head_tile_ok(const QrowParams& p, int x_dtype, int64_t M) {
+  const int es = x_dtype == QS_F32 ? 4 : 2;
+  return M >= (x_dtype == QS_F32 ? 5 : 3) && p.K % 128 == 0 && p.K >= 512 && (int64_t)16 * p.K * es <= 144 * 1024 && p.ldx * es % 16 == 0 &&
+         aligned(p.x, 16) && aligned(p.lin[0].codes, 16);
+}
+
+// Workgroups of k_head_top2 (8 waves of 16-row tiles): as many as are resident, two per CU
+// while two copies of the activations fit its LDS.
+int head_grid(int rows, size_t lds) {
+  const int64_t n = cdiv(rows, 8 * 16), cap = lds <= 80 * 1024 ? 512 : 256;
+  return (int)(n < cap ? n : cap);
+}
+
+template <int XT>
+void launch_head(const QrowParams& q, int rows, int start_row, float* pv, int* pi, int grid, hipStream_t s) {
+  const size_t lds = (size_t)16 * q.K * (XT == QS_F32 ? 4 : 2);
+  const int C = q.K / 64;
+  if (C % 8 == 0) hipLaunchKernelGGL((k_head_top2<XT, 8>), dim3(grid), dim3(512), lds, s, q, rows, start_row, pv, pi);
+  else if (C % 4 == 0) hipLaunchKernelGGL((k_head_top2<XT, 4>), dim3(grid), dim3(512), lds, s, q, rows, start_row, pv, pi);
+  else hipLaunchKernelGGL((k_head_top2<XT, 2>), dim3(grid), dim3(512), lds, s, q, rows, start_row, pv, pi);
+}
+
 // Launches of the top-2 search for validated arguments, M >= 1, with the per-block
 // candidates in `workspace` (at least qs_qrow_top2_workspace_bytes(M, row_count) bytes).
 // Every candidate slot the reduce reads is written by the search first, so the workspace
@@ -2029,7 +2189,18 @@ int top2_launch(const void* x, int x_dtype, int64_t ldx, const int8_t* codes, co
   p.lin[0] = QrowLin{codes, scales, nullptr, 0, (int)row_count, 0};
   const int rows = (int)row_count;
   int C;
-  if (valu_eligible(p, x_dtype)) {
+  if (head_tile_ok(p, x_dtype, M)) {
+    const int g = head_grid(rows, (size_t)16 * K * es);  // at most top2_blocks(): the candidates fit the workspace
+    C = 2 * g;
+    for (int64_t m0 = 0; m0 < M; m0 += 16) {
+      QrowParams q = p;
+      q.M = (int)((M - m0) < 16 ? (M - m0) : 16);
+      q.x = static_cast<const char*>(x) + m0 * ldx * es;
+      if (x_dtype == QS_F32) launch_head<QS_F32>(q, rows, (int)start_row, pv + m0 * C, pi + m0 * C, g, s);
+      else if (x_dtype == QS_BF16) launch_head<QS_BF16>(q, rows, (int)start_row, pv + m0 * C, pi + m0 * C, g, s);
+      else launch_head<QS_F16>(q, rows, (int)start_row, pv + m0 * C, pi + m0 * C, g, s);
+    }
+  } else if (valu_eligible(p, x_dtype)) {
     const int mb = valu_mb(x_dtype, K, M);
     C = 2 * top2_grid(rows);
     for (int64_t m0 = 0; m0 < M; m0 += mb) {
