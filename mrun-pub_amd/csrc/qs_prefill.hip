@@ -1,7 +1,7 @@
 // qrow linears for many activation rows (prefill) on gfx950: W8A16 and fp32.
 //
 // Kernels
-//   k_prefill<P, MT, NT, WN, WK, D, XT> : one workgroup = a tile of 16 * MT activation rows
+//   k_prefill<P, MT, NT, WN, WK, XT> : one workgroup = a tile of 16 * MT activation rows
 //                               and 16 * NT * WN weight rows (of P planes; P = 2 pairs the
 //                               gate and up rows of a SwiGLU) x one K slice.
 //   k_prefill_reduce<P, XT>   : the K slices' fp32 partial sums added in slice order, and the
@@ -86,11 +86,12 @@ constexpr int kPfFlush = 6;
 // before: one launch of the one-row VALU kernel per row), 64 x 8960 x 1536 155 -> 29 us,
 // 9 x 4096 x 1024 15.0 -> 8.4 us.  Error against 64-bit sums 1.0e-7..1.2e-7 (VALU: 1.0e-7 at
 // K = 1024 to 2.3e-7 at K = 8960).
-template <int P, int MT, int NT, int WN, int WK, int D, int XT>
+template <int P, int MT, int NT, int WN, int WK, int XT>
 __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
   constexpr bool F32 = XT == QS_F32;
   typedef Half<XT == QS_F16> H;
   typedef typename H::vec hvec;
+  constexpr int D = 2;  // iterations in flight
   constexpr int NW = WN * WK;
   constexpr int TM = 16 * MT, TN = 16 * NT * WN;
   constexpr int ES = F32 ? 4 : 2;
@@ -187,13 +188,13 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
                                                          t < T ? (t0 + t) * 64 : 0, 0));
   };
 
-  f32x4 acc[P][NT][MT];
+  f32x4 acc[P][NT][MT], sum[P][NT][MT];
 #pragma unroll
   for (int pl = 0; pl < P; ++pl)
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) acc[pl][j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int m = 0; m < MT; ++m) acc[pl][j][m] = sum[pl][j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // iteration i from stage st; its weight registers take the weights of iteration i + D as
   // soon as they are dequantized.  16-bit: the lane's 16 codes make two MFMA fragments.
@@ -232,10 +233,6 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
   // accumulators: short chains, as exact as the row's sum over a wave's lanes.
   auto mul32 = [&](i32x4 (&w)[P][NT], int i, int st) {
     const uint8_t* xs = lds + st * STAGE + wk * SUB + col * ROW;
-    i32x4 wv[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) wv[j] = w[0][j];
-    load_w(w, i + D);
     f32x4 part[2][NT][MT];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -244,7 +241,7 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
       for (int m = 0; m < MT; ++m) x[m] = *reinterpret_cast<const f32x4*>(xs + 16 * ((4 * grp + c) ^ sw) + 16 * ROW * m);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const int d = wv[j][c];
+        const int d = w[0][j][c];
         const float wf[4] = {sbyte_f32<0>(d) * sc[0][j], sbyte_f32<1>(d) * sc[0][j], sbyte_f32<2>(d) * sc[0][j],
                              sbyte_f32<3>(d) * sc[0][j]};
 #pragma unroll
@@ -260,7 +257,8 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) acc[0][j][m] += part[0][j][m] + part[1][j][m];
+      for (int m = 0; m < MT; ++m) sum[0][j][m] += part[0][j][m] + part[1][j][m];
+    load_w(w, i + D);
   };
   auto mul = [&](i32x4 (&w)[P][NT], int i, int st) {
     if constexpr (F32) mul32(w, i, st);
@@ -275,40 +273,53 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
 #pragma unroll
   for (int d = 0; d < D; ++d) {
     copy_x(d, d);
+    __builtin_amdgcn_sched_barrier(0);
     load_w(w[d], d);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  f32x4 sum[P][NT][MT];
-#pragma unroll
-  for (int pl = 0; pl < P; ++pl)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) sum[pl][j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // The weight registers of an even and an odd iteration alternate in the loop body, and
+  // every exit leaves it whole: the compiler then counts the loads still in flight exactly
+  // (paths that join with another order of requests make it wait for the newest ones).
   auto flush = [&]() {
+    if constexpr (!F32) {
 #pragma unroll
-    for (int pl = 0; pl < P; ++pl)
+      for (int pl = 0; pl < P; ++pl)
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          sum[pl][j][m] += acc[pl][j][m];
-          acc[pl][j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+          for (int m = 0; m < MT; ++m) {
+            sum[pl][j][m] += acc[pl][j][m];
+            acc[pl][j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+    }
   };
   int st = 0;
-  for (int i = 0; i < I;) {
-    for (int f = 0; f < kPfFlush && i < I; f += D) {
-#pragma unroll
-      for (int d = 0; d < D; ++d) {
-        pf_wait_barrier<(D - 1) * GROUP>();
-        copy_x(i + D, st == 0 ? D : st - 1);
-        mul(w[d], i, st);
-        st = st == D ? 0 : st + 1;
-        if (++i >= I) break;
-      }
+  auto step = [&](int d, int i) {
+    pf_wait_barrier<(D - 1) * GROUP>();
+    copy_x(i + D, st == 0 ? D : st - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mul(w[d], i, st);
+    st = st == D ? 0 : st + 1;
+  };
+  static_assert(kPfFlush == 6, "steps between flushes below");
+  for (int i = 0;;) {
+    step(0, i);
+    if (++i >= I) break;
+    step(1, i);
+    if (++i >= I) break;
+    if constexpr (!F32) {
+      step(0, i);
+      if (++i >= I) break;
+      step(1, i);
+      if (++i >= I) break;
+      step(0, i);
+      if (++i >= I) break;
+      step(1, i);
+      if (++i >= I) break;
+      flush();
     }
-    flush();
   }
+  flush();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies past the slice
 
   // the WK parts are added in order through LDS, one 16-row block of weights at a time
@@ -506,7 +517,7 @@ void pf_launch(const PfParams& p, int shape, hipStream_t s) {
 #define QS_PF(K_)                                                                                               \
   if (shape == K_) {                                                                                            \
     constexpr PfShape h = kPfShapes[K_];                                                                        \
-    hipLaunchKernelGGL((k_prefill<P, h.MT, h.NTP / P, h.WN, h.WK, 2, XT>), grid, dim3(h.WN * h.WK * 64), 0, s, p); \
+    hipLaunchKernelGGL((k_prefill<P, h.MT, h.NTP / P, h.WN, h.WK, XT>), grid, dim3(h.WN * h.WK * 64), 0, s, p); \
   }
   if constexpr (XT == QS_F32) {
     QS_PF(4) QS_PF(5)
