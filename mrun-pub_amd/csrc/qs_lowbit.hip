@@ -16,47 +16,18 @@
 // and y += scale * (R - (OFF + z) * S0).  fp32 activations are split exactly into three
 // bf16 terms (x = h + m + l) that run as three activation rows and are summed at the end.
 //   k_lowbit_valu  decode (M <= 2 bf16 rows): one wave per weight row, v_dot2_f32_bf16
+//   k_lowbit_gemm  (qs_lowbit_gemm.hip) more than 16 bf16 or 5 fp32 rows, one launch
 //   k_lowbit_gk    3..16 bf16 rows, one launch: v_mfma_f32_16x16x32_bf16 per group, a
 //                  quarter group per lane, K split over the waves of a workgroup
 //   k_lowbit_slot  M <= 16 fp32 rows (split into bf16 terms): one whole group per lane
 //   k_lowbit_mfma  any aligned-to-4 layout (fallback), four lanes per group
 //   k_lowbit_any   every other layout (any group size, a short last group, unaligned
 //                  rows): one wave per weight row, scalar decode
-#include "qs_common.h"
+#include "qs_lowbit.h"
 
 #include <limits.h>
 
 namespace qs {
-
-struct LowbitParams {
-  const uint16_t* x;   // bf16 [M, K] (M <= 16)
-  int64_t ldx;
-  const float* s0;     // [M, ng] group sums of x
-  const uint8_t* packed;
-  int64_t row_bytes;
-  const void* scales;  // [N, ng] f32 or f16
-  const void* zeros;   // [N, ng] f16/f32, nullable
-  int scale_f16, zero_f16;
-  float offset;        // used when zeros == nullptr
-  float* y;            // [M, N]
-  int64_t ldy;
-  int M, N, K, ng;
-  uint32_t pair_mask, pair_base;  // code-pair -> bf16x2 (OFF + c) masks, set by pair_consts()
-};
-
-// (t * spread) & mask | base turns the 2*BITS-bit code pair t into two bf16 (OFF + c).
-// mask/base travel as kernel arguments (scalar registers) so that the and/or is a single
-// v_bitop3_b32 (table 0xEA = (a & b) | c).
-template <int BITS>
-__device__ __forceinline__ uint32_t pair_bf16(uint32_t t, uint32_t mask, uint32_t base) {
-  constexpr uint32_t spread = BITS == 3 ? 0x20010u : 0x80020u;
-  return __builtin_amdgcn_bitop3_b32(t * spread, mask, base, 0xEA);
-}
-
-inline void pair_consts(LowbitParams& p, int bits) {
-  p.pair_mask = bits == 3 ? 0x00700070u : 0x00600060u;
-  p.pair_base = bits == 3 ? 0x41004100u : 0x40804080u;
-}
 
 // Lane code extraction: the lane's G/4 codes (BITS*G/4 bits, at a 2- or 4-byte aligned
 // offset) are returned as a 64/96-bit little-endian field.
@@ -97,18 +68,6 @@ __device__ __forceinline__ void load_codes(const uint8_t* p, uint32_t (&f)[3]) {
     }
     f[2] = 0;
   }
-}
-
-// 2 codes starting at bit position bp of the field -> packed bf16 pair (OFF + c).
-template <int BITS>
-__device__ __forceinline__ uint32_t code_pair(const uint32_t (&f)[3], int bp, uint32_t mask, uint32_t base) {
-  const int w = bp >> 5, o = bp & 31;
-  uint32_t t;
-  if (o + 2 * BITS <= 32)
-    t = __builtin_amdgcn_ubfe(f[w], o, 2 * BITS);
-  else
-    t = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(f[w + 1], f[w], o), 0, 2 * BITS);
-  return pair_bf16<BITS>(t, mask, base);  // int3: 8 + c at bits 4-6 / 20-22; int2: 4 + c at 5-6 / 21-22
 }
 
 template <int BITS, int G, int KW>
@@ -1178,6 +1137,13 @@ int check_lowbit(const void* packed, int64_t row_bytes, const void* scales, int 
   return QS_OK;
 }
 
+}  // namespace
+
+void launch_lowbit_prep(const void* x, int x_dtype, int64_t ldx, int M, int K, uint16_t* xb, hipStream_t s) {
+  hipLaunchKernelGGL(k_lowbit_prep, dim3((unsigned)cdiv((int64_t)M * K, 256)), dim3(256), 0, s, x, x_dtype, ldx, M, K, xb);
+}
+
+namespace {
 // the tiled kernels' layout: G 64 or 128, whole groups, 4-byte aligned rows
 bool tiled_layout(const void* packed, int64_t row_bytes, int G, int64_t K) {
   return (G == 64 || G == 128) && K % G == 0 && row_bytes % 4 == 0 && aligned(packed, 4);
@@ -1188,6 +1154,15 @@ bool tiled_layout(const void* packed, int64_t row_bytes, int G, int64_t K) {
 using namespace qs;
 
 static constexpr int kLowbitMaxSplit = 8;  // K splits of k_lowbit_slot (partial-sum planes)
+
+// Workspace of the kernels that take one batch of rows at a time, whatever M is.
+static size_t lowbit_base_workspace(int64_t N, int64_t K, int group_size) {
+  const int64_t ng = group_size > 0 ? K / group_size : 0;
+  const size_t xb = ((size_t)16 * K * 2 + 255) / 256 * 256;
+  const size_t s0 = ((size_t)16 * ng * 4 + 255) / 256 * 256;
+  const size_t y3 = (size_t)kLowbitMaxSplit * 16 * N * 4;
+  return xb + s0 + y3;
+}
 
 extern "C" int qs_lowbit_gemv(const void* x, int x_dtype, int64_t ldx, const uint8_t* packed,
                               int64_t row_bytes, const void* scales, int scale_dtype,
@@ -1231,12 +1206,19 @@ extern "C" int qs_lowbit_gemv(const void* x, int x_dtype, int64_t ldx, const uin
   const int rows_per_x = x_dtype == QS_F32 ? 3 : 1;
   const int mb = x_dtype == QS_F32 ? 5 : 16;  // activation rows per MFMA tile
   const int ng = (int)(K / group_size);
-  const size_t need = qs_lowbit_workspace_bytes(x_dtype, M, N, K, group_size);
+  const size_t need = lowbit_base_workspace(N, K, group_size);  // more lets more rows share a launch
   if (!workspace || workspace_bytes < need)
     return fail(QS_ERR_INVALID, "lowbit_gemv: workspace of %zu bytes required", need);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int cb = bits * group_size / 8;
-  (void)cb;
+  // More rows than one k_lowbit_gk (16 bf16) or k_lowbit_slot (5 fp32) launch: one launch over
+  // all rows.  17 rows already gain (int3 G = 64: 4096 x 11008 29 -> 17 us, 11008 x 4096
+  // 26 -> 21; int2 G = 64 11008 x 4096 level at 20).
+  if (M > mb && ((scale_dtype == QS_F16 && zeros && zero_dtype == QS_F16) || (scale_dtype == QS_F32 && !zeros))) {
+    const LowbitGemm a{x, x_dtype, ldx, packed, row_bytes, scales, zeros, scale_dtype == QS_F16, offset, bits,
+                       group_size, y, ldy, M, N, K};
+    st = run_lowbit_gemm(a, workspace, workspace_bytes, s);
+    if (st != QS_ERR_UNSUPPORTED) return st;
+  }
   const bool tiled = row_bytes % 8 == 0 && aligned(packed, 8) && aligned(workspace, 16);
   // workspace: bf16 rows [16, K] | s0 [16, ng] | partial sums [kLowbitMaxSplit, 16, N]
   uint8_t* ws = static_cast<uint8_t*>(workspace);
@@ -1293,7 +1275,8 @@ extern "C" int qs_lowbit_gemv(const void* x, int x_dtype, int64_t ldx, const uin
     }
   }
   {
-    // 3..16 bf16 rows (and any bf16 M in chunks of 16): the single-launch group-MFMA kernel
+    // 3..16 bf16 rows (and any M that k_lowbit_gemm refuses, in chunks of 16): the
+    // single-launch group-MFMA kernel
     const bool layout = (scale_dtype == QS_F16 && zeros && zero_dtype == QS_F16) || (scale_dtype == QS_F32 && !zeros);
     const int ngr = group_size == 64 ? kGkGroupsLong<64> : kGkGroupsLong<128>;
     const int waves = (int)cdiv(ng, ngr);  // the long form's count bounds both
@@ -1402,13 +1385,10 @@ extern "C" int qs_lowbit_gemv(const void* x, int x_dtype, int64_t ldx, const uin
 }
 
 extern "C" size_t qs_lowbit_workspace_bytes(int x_dtype, int64_t M, int64_t N, int64_t K, int group_size) {
-  (void)M;
-  (void)x_dtype;
-  const int64_t ng = group_size > 0 ? K / group_size : 0;
-  const size_t xb = ((size_t)16 * K * 2 + 255) / 256 * 256;
-  const size_t s0 = ((size_t)16 * ng * 4 + 255) / 256 * 256;
-  const size_t y3 = (size_t)kLowbitMaxSplit * 16 * N * 4;
-  return xb + s0 + y3;
+  const size_t base = lowbit_base_workspace(N, K, group_size);
+  if (M <= (x_dtype == QS_F32 ? 5 : 16)) return base;
+  const size_t many = lowbit_gemm_workspace(x_dtype, M, N, K, group_size);
+  return many > base ? many : base;
 }
 
 extern "C" int qs_lowbit_dequant(const uint8_t* packed, int64_t row_bytes, const void* scales,
