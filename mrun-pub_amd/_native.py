@@ -13,6 +13,7 @@ invalid arguments -> ``ValueError``; unsupported / runtime failures -> ``Runtime
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -149,9 +150,29 @@ def call(name: str, *args) -> None:
     check(getattr(load(), name)(*args), name)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(device: torch.device) -> int:
     """hipStream_t of torch's current stream on ``device`` (as an int)."""
+    # the raw handle, without a Stream object around it (0.1 us against 2.1)
+    if device.index is not None and _raw_stream is not None:
+        return _raw_stream(device.index)
     return int(torch.cuda.current_stream(device).cuda_stream)
+
+
+def inference(fn):
+    """``torch.inference_mode()`` for an operator, as a guard that an enclosing inference mode
+    makes unnecessary and that is entered directly otherwise (0.6 us less per call)."""
+
+    @functools.wraps(fn)
+    def run(*args, **kwargs):
+        if torch.is_inference_mode_enabled():
+            return fn(*args, **kwargs)
+        with torch._C._InferenceMode(True):
+            return fn(*args, **kwargs)
+
+    return run
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -160,19 +181,19 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
     """All tensors must live on one HIP device; returns it."""
-    device = None
+    first, index = None, -1
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ValueError("QStore HIP operators require tensors on a HIP (cuda) device")
-        if device is None:
-            device = t.device
-        elif t.device != device:
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
             raise ValueError("QStore HIP operator tensors must share one device")
-    if device is None:
+    if first is None:
         raise ValueError("no device tensor given")
-    return device
+    return first.device
 
 
 def pointer_array(values: list[int]) -> ctypes.Array:

@@ -28,7 +28,7 @@ def _check(W: torch.Tensor) -> tuple[int, int, torch.device]:
     return int(W.shape[0]), int(W.shape[1]), device
 
 
-@torch.inference_mode()
+@nat.inference
 def quant_row_int8(W: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Per-row symmetric int8: ``(q int8 [out, in], scale float32 [out])``."""
     n, k, device = _check(W)
@@ -55,13 +55,13 @@ def _lowbit(W: torch.Tensor, bits: int, G: int) -> tuple[torch.Tensor, torch.Ten
     return packed, scales
 
 
-@torch.inference_mode()
+@nat.inference
 def quant_row_int3(W: torch.Tensor, G: int = GROUP) -> tuple[torch.Tensor, torch.Tensor]:
     """Group-wise symmetric int3: ``(packed uint8 [out, ceil(in*3/8)], scales [out, ceil(in/G)])``."""
     return _lowbit(W, 3, G)
 
 
-@torch.inference_mode()
+@nat.inference
 def quant_row_int2(W: torch.Tensor, G: int = GROUP) -> tuple[torch.Tensor, torch.Tensor]:
     """Group-wise TWN ternary int2: ``(packed uint8 [out, ceil(in*2/8)], scales [out, ceil(in/G)])``."""
     return _lowbit(W, 2, G)

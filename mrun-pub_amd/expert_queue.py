@@ -154,7 +154,7 @@ def _compile(rows: int, top_k: int, num_experts: int, experts: torch.Tensor, wei
                            p_deadlines, starts, counts)
 
 
-@torch.inference_mode()
+@nat.inference
 def build_expert_queue(top_indices: torch.Tensor, top_weights: torch.Tensor, *, num_experts: int,
                        epochs: torch.Tensor, deadlines: torch.Tensor) -> ExpertQueuePlan:
     """Validated, stable expert-major plan of ``[rows, top_k]`` router output
@@ -174,7 +174,7 @@ def build_expert_queue(top_indices: torch.Tensor, top_weights: torch.Tensor, *, 
     return plan
 
 
-@torch.inference_mode()
+@nat.inference
 def build_expert_queue_flat(token_ids: torch.Tensor, expert_ids: torch.Tensor, route_slots: torch.Tensor,
                             coefficients: torch.Tensor, *, num_rows: int, num_experts: int, top_k: int,
                             epochs: torch.Tensor, deadlines: torch.Tensor,
@@ -230,7 +230,7 @@ def build_expert_queue_flat(token_ids: torch.Tensor, expert_ids: torch.Tensor, r
     return plan
 
 
-@torch.inference_mode()
+@nat.inference
 def build_expert_queue_device(top_indices: torch.Tensor, top_weights: torch.Tensor, *, num_experts: int,
                               epochs: torch.Tensor, deadlines: torch.Tensor, block: int = 256) -> ExpertQueuePlan:
     """Plan of router output that upstream code already validated (expert_queue.py:401-484):
@@ -277,7 +277,7 @@ def _scatter(plan: ExpertQueuePlan, expert_outputs: torch.Tensor, active_epochs:
     return reduced, valid.view(torch.bool)
 
 
-@torch.inference_mode()
+@nat.inference
 def scatter_committed(plan: ExpertQueuePlan, expert_outputs: torch.Tensor, *,
                       active_epochs: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """``(reduced [rows, hidden] fp32, valid [assignments] bool)``: packets whose epoch equals
@@ -285,7 +285,7 @@ def scatter_committed(plan: ExpertQueuePlan, expert_outputs: torch.Tensor, *,
     return _scatter(plan, expert_outputs, active_epochs)
 
 
-@torch.inference_mode()
+@nat.inference
 def scatter_committed_device(plan: ExpertQueuePlan, expert_outputs: torch.Tensor, *, active_epochs: torch.Tensor,
                              block_assignments: int = 128,
                              block_hidden: int = 32) -> tuple[torch.Tensor, torch.Tensor]:

@@ -65,7 +65,7 @@ def _check(page: LowbitPage) -> None:
         raise ValueError("zeros must match scales in shape and be float32/float16")
 
 
-@torch.inference_mode()
+@nat.inference
 def lowbit_dequant(page: LowbitPage) -> torch.Tensor:
     """fp32 ``[out, in]`` weight ``(float(code) - zero) * scale`` (qstore.py:441-456)."""
     _check(page)
@@ -80,7 +80,7 @@ def lowbit_dequant(page: LowbitPage) -> torch.Tensor:
     return out
 
 
-@torch.inference_mode()
+@nat.inference
 def lowbit_matmul(page: LowbitPage, x: torch.Tensor, *, row_stable: bool = False) -> torch.Tensor:
     """``x[..., in] @ W.T`` in fp32 (``QStoreInt3.matmul`` contract), fp32 ``[..., out]``.
 
@@ -93,14 +93,14 @@ def lowbit_matmul(page: LowbitPage, x: torch.Tensor, *, row_stable: bool = False
     if int(x.shape[-1]) != K:
         raise ValueError("activation width does not match the packed block")
     device = nat.require_device(page.packed, page.scales, page.zeros, x)
-    x2 = x.reshape(-1, K)
+    x2 = x if x.ndim == 2 else x.reshape(-1, K)
     if x2.dtype not in (torch.bfloat16, torch.float32):
         x2 = x2.to(torch.float32)
     x2 = x2.contiguous()
     M, N = int(x2.shape[0]), page.out_features
     y = torch.empty((M, N), dtype=torch.float32, device=device)
     _gemv_into(page, x2, y, N, row_stable=row_stable)
-    return y.reshape(*x.shape[:-1], N)
+    return y if x.ndim == 2 else y.reshape(*x.shape[:-1], N)
 
 
 def _gemv_into(page: LowbitPage, x2: torch.Tensor, y: torch.Tensor, ldy: int, *, row_stable: bool) -> None:

@@ -39,7 +39,7 @@ def _align(n: int, a: int = 4096) -> int:
 # ---- router ------------------------------------------------------------------------------
 
 
-@torch.inference_mode()
+@nat.inference
 def route_topk(
     logits: torch.Tensor, top_k: int, *, norm_topk: bool = True, out_dtype: torch.dtype = torch.bfloat16
 ) -> tuple[torch.Tensor, torch.Tensor]:
@@ -149,7 +149,7 @@ def _compact_route_with_inverse(top_indices, top_weights, selected_experts):
 # ---- reducer -------------------------------------------------------------------------------
 
 
-@torch.inference_mode()
+@nat.inference
 def stable_route_reduce(
     expert_output: torch.Tensor,
     coefficients: torch.Tensor,
@@ -214,7 +214,7 @@ def stable_route_reduce(
 # ---- grouped GEMM --------------------------------------------------------------------------
 
 
-@torch.inference_mode()
+@nat.inference
 def quantize_rows(source: torch.Tensor, rows: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """int8 codes and fp32 scales of ``source[rows]`` (per-row absmax/127, W8A8 recipe)."""
     device = nat.require_device(source, rows)
@@ -257,7 +257,7 @@ def _grouped_contract(rows_q, weights, weight_scales, starts, counts, group_slot
     return logical, n_out, contraction
 
 
-@torch.inference_mode()
+@nat.inference
 def grouped_int8_mm(
     rows_q: torch.Tensor,
     row_scales: torch.Tensor,
@@ -312,7 +312,7 @@ def grouped_int8_mm(
     return out, IMPL_GROUPED
 
 
-@torch.inference_mode()
+@nat.inference
 def grouped_w8a16_mm(
     rows: torch.Tensor,
     weights: torch.Tensor,
@@ -490,7 +490,7 @@ class Int8ExpertBackend:
             ids = self._experts[key] = torch.arange(E, device=device)
         return ids
 
-    @torch.inference_mode()
+    @nat.inference
     def moe(
         self,
         layer: int,

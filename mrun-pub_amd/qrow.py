@@ -77,7 +77,7 @@ def _check_codes(codes: torch.Tensor, scales: torch.Tensor) -> tuple[int, int]:
     return int(codes.shape[0]), int(codes.shape[1])
 
 
-@torch.inference_mode()
+@nat.inference
 def qrow_dequant(
     codes: torch.Tensor, scales: torch.Tensor, dtype: torch.dtype = torch.float32
 ) -> torch.Tensor:
@@ -113,7 +113,7 @@ def normalize_row_ids(ids, n_rows: int):
     return np.where(idx < 0, idx + n_rows, idx), idx.shape
 
 
-@torch.inference_mode()
+@nat.inference
 def qrow_embed_rows(codes: torch.Tensor, scales: torch.Tensor, ids) -> torch.Tensor:
     """fp32 rows ``float(codes[ids]) * scales[ids]`` with shape ``[*ids.shape, in]``
     (the qrow branch of ``QStore.embed_rows``, qstore.py:1099-1128)."""
@@ -126,6 +126,19 @@ def qrow_embed_rows(codes: torch.Tensor, scales: torch.Tensor, ids) -> torch.Ten
         nat.call("qs_qrow_dequant_rows", nat.ptr(codes), nat.ptr(scales), n, k, nat.ptr(rows),
                  int(rows.numel()), nat.ptr(out), nat.stream_of(device))
     return out.reshape(*shape, k)
+
+
+def _rows(x: torch.Tensor, k: int) -> torch.Tensor:
+    """``x[..., k]`` as contiguous rows ``[m, k]`` (``x`` itself when it is that already)."""
+    if x.ndim == 2 and x.shape[1] == k and x.is_contiguous():
+        return x
+    flat = x.reshape(-1, k)
+    return flat if flat.is_contiguous() else flat.contiguous()
+
+
+def _like_rows(y: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """``y[m, n]`` in the leading shape of ``x``."""
+    return y if x.ndim == 2 and y.shape[0] == x.shape[0] else y.reshape(*x.shape[:-1], y.shape[1])
 
 
 def _out_buffer(out: torch.Tensor | None, m: int, n: int, dtype: torch.dtype, device) -> torch.Tensor:
@@ -215,7 +228,7 @@ def _run_many(kind: str, x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch
         ws_bytes = int(lib.qs_qrow_batched_workspace_bytes(m, len(ns), n_arr, k, int(swiglu)))
     else:
         ws_bytes = int(lib.qs_qrow_prefill_workspace_bytes(xdt, m, len(ns), n_arr, k, int(swiglu)))
-    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
     if swiglu:
         (gc, gs), (uc, us) = pages
         nat.call(f"qs_qrow_swiglu_{kind}", nat.ptr(x2), k, nat.ptr(gc), nat.ptr(gs), nat.ptr(uc), nat.ptr(us),
@@ -226,7 +239,7 @@ def _run_many(kind: str, x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch
                  nat.pointer_array([nat.ptr(o) for o in outs]), n_arr, n_arr, m, k, nat.ptr(ws), ws_bytes, stream)
 
 
-@torch.inference_mode()
+@nat.inference
 def qrow_matmul(
     codes: torch.Tensor, scales: torch.Tensor, x: torch.Tensor, *, row_stable: bool = False,
     out: torch.Tensor | None = None,
@@ -246,9 +259,7 @@ def qrow_matmul(
     if x.ndim < 1 or int(x.shape[-1]) != k:
         raise ValueError("activation width does not match compact qrow page")
     device = nat.require_device(codes, scales, x)
-    flat = x.reshape(-1, k)
-    if not flat.is_contiguous():
-        flat = flat.contiguous()
+    flat = _rows(x, k)
     m = int(flat.shape[0])
     y = _out_buffer(out, m, n, x.dtype, device)
     if m > 1 and not row_stable and _batched_eligible(flat, [codes]):
@@ -270,10 +281,10 @@ def qrow_matmul(
             k,
             nat.stream_of(device),
         )
-    return y.reshape(*x.shape[:-1], n)
+    return _like_rows(y, x)
 
 
-@torch.inference_mode()
+@nat.inference
 def qrow_matmul_multi(
     pages: list[tuple[torch.Tensor, torch.Tensor]], x: torch.Tensor,
     out: list[torch.Tensor] | None = None,
@@ -289,7 +300,7 @@ def qrow_matmul_multi(
     if x.dtype not in _ACT_DTYPES:
         raise ValueError(f"activation dtype {x.dtype} not supported")
     device = nat.require_device(x, *[t for p in pages for t in p])
-    flat = x.reshape(-1, k).contiguous()
+    flat = _rows(x, k)
     m = int(flat.shape[0])
     if out is not None and len(out) != len(pages):
         raise ValueError("one output buffer per linear")
@@ -314,7 +325,7 @@ def qrow_matmul_multi(
             k,
             nat.stream_of(device),
         )
-    return [o.reshape(*x.shape[:-1], o.shape[1]) for o in outs]
+    return [_like_rows(o, x) for o in outs]
 
 
 def _validate_block_m(block_m: int) -> None:
@@ -323,7 +334,7 @@ def _validate_block_m(block_m: int) -> None:
         raise ValueError("block_m must be one of 16, 32, or 64")
 
 
-@torch.inference_mode()
+@nat.inference
 def fused_qrow_matmul(
     page: CompactQRowPage,
     activations: torch.Tensor,
@@ -366,7 +377,7 @@ def _validate_paired_qrow_pages(
         raise ValueError("paired compact qrow pages and activations must use one device")
 
 
-@torch.inference_mode()
+@nat.inference
 def fused_qrow_swiglu(
     gate_page: CompactQRowPage,
     up_page: CompactQRowPage,
@@ -381,7 +392,7 @@ def fused_qrow_swiglu(
     return qrow_swiglu_into(gate_page, up_page, activations), IMPL_SWIGLU
 
 
-@torch.inference_mode()
+@nat.inference
 def qrow_swiglu_into(gate_page: CompactQRowPage, up_page: CompactQRowPage, activations: torch.Tensor,
                      out: torch.Tensor | None = None) -> torch.Tensor:
     """The paired SwiGLU of :func:`fused_qrow_swiglu`, optionally into a preallocated bf16
@@ -390,7 +401,7 @@ def qrow_swiglu_into(gate_page: CompactQRowPage, up_page: CompactQRowPage, activ
     n, k = _check_codes(gate_page.codes, gate_page.scales)
     _check_codes(up_page.codes, up_page.scales)
     device = nat.require_device(activations, gate_page.codes)
-    flat = activations.reshape(-1, k).contiguous()
+    flat = _rows(activations, k)
     m = int(flat.shape[0])
     y = _out_buffer(out, m, n, torch.bfloat16, device)
     if m > 1 and _batched_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
@@ -413,7 +424,7 @@ def qrow_swiglu_into(gate_page: CompactQRowPage, up_page: CompactQRowPage, activ
             k,
             nat.stream_of(device),
         )
-    return y.reshape(*activations.shape[:-1], n)
+    return _like_rows(y, activations)
 
 
 # ---- head: fused top-2 and fp32 candidate rerank ----------------------------------------------
@@ -438,7 +449,7 @@ def _check_head(page: CompactQRowPage, activations: torch.Tensor) -> None:
         raise ValueError("head page and activations must use one device")
 
 
-@torch.inference_mode()
+@nat.inference
 def fused_qrow_top2(
     page: CompactQRowPage,
     activations: torch.Tensor,
@@ -464,9 +475,7 @@ def fused_qrow_top2(
         raise ValueError(f"activation dtype {activations.dtype} not supported")
     n, k = _check_codes(page.codes, page.scales)
     device = nat.require_device(activations, page.codes)
-    flat = activations.reshape(-1, k)
-    if not flat.is_contiguous():
-        flat = flat.contiguous()
+    flat = _rows(activations, k)
     m = int(flat.shape[0])
     out_i = torch.empty((m, 2), dtype=torch.int32, device=device)
     out_v = torch.empty((m, 2), dtype=torch.float32, device=device)
@@ -501,9 +510,7 @@ def _rerank(page: CompactQRowPage, activations: torch.Tensor, candidate_indices:
         raise ValueError(f"activation dtype {activations.dtype} not supported")
     n, k = _check_codes(page.codes, page.scales)
     device = nat.require_device(activations, page.codes)
-    flat = activations.reshape(-1, k)
-    if not flat.is_contiguous():
-        flat = flat.contiguous()
+    flat = _rows(activations, k)
     m = int(flat.shape[0])
     cand = candidate_indices.reshape(m, -1).to(torch.long).contiguous()
     c = int(cand.shape[1])
@@ -523,7 +530,7 @@ def _rerank(page: CompactQRowPage, activations: torch.Tensor, candidate_indices:
     return out_i.reshape(shape), out_v.reshape(shape)
 
 
-@torch.inference_mode()
+@nat.inference
 def rerank_qrow_candidates_fp32(
     page: CompactQRowPage, activations: torch.Tensor, candidate_indices: torch.Tensor
 ) -> tuple[torch.Tensor, torch.Tensor]:
@@ -532,7 +539,7 @@ def rerank_qrow_candidates_fp32(
     return _rerank(page, activations, candidate_indices, validate_candidate_bounds=True)
 
 
-@torch.inference_mode()
+@nat.inference
 def fused_qrow_reranked_argmax(
     page: CompactQRowPage,
     activations: torch.Tensor,

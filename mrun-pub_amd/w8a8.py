@@ -36,7 +36,7 @@ def _check_weight(q_w: torch.Tensor, sc_w: torch.Tensor) -> tuple[int, int]:
     return int(q_w.shape[0]), int(q_w.shape[1])
 
 
-@torch.inference_mode()
+@nat.inference
 def _int8_gemm(q_x: torch.Tensor, q_w: torch.Tensor, use_int_mm: bool = True) -> torch.Tensor:
     """``[T,in] int8 @ [out,in] int8^T -> [T,out] int32`` (w8a8.py:33-64), exact.
 
@@ -59,7 +59,7 @@ def _int8_gemm(q_x: torch.Tensor, q_w: torch.Tensor, use_int_mm: bool = True) ->
     return acc
 
 
-@torch.inference_mode()
+@nat.inference
 def quantize_activation(
     x: torch.Tensor, keep: torch.Tensor | None = None
 ) -> tuple[torch.Tensor, torch.Tensor]:
@@ -94,7 +94,7 @@ def _fused_front_end_ok(x2: torch.Tensor, protect_k: int, inn: int) -> bool:
             and x2.data_ptr() % 16 == 0)
 
 
-@torch.inference_mode()
+@nat.inference
 def w8a8_matmul(
     q_w: torch.Tensor,
     sc_w: torch.Tensor,
@@ -119,7 +119,7 @@ def w8a8_matmul(
     if out_dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("out_dtype must be float32 or bfloat16")
     device = nat.require_device(q_w, sc_w, x)
-    x2 = x.reshape(-1, inn).contiguous()
+    x2 = (x if x.ndim == 2 else x.reshape(-1, inn)).contiguous()
     T = int(x2.shape[0])
     y = torch.empty((T, out), dtype=out_dtype, device=device)
     if T == 0:
@@ -132,16 +132,18 @@ def w8a8_matmul(
     if protect_idx is None and protect_k > 0 and _fused_front_end_ok(x2, protect_k, inn):
         # column maxima, then selection + quantization + side operands in one launch
         k = min(int(protect_k), inn)
-        colws = torch.empty(((T + 1023) // 1024) * inn, dtype=torch.float32, device=device)
-        q_x = torch.empty((T, inn), dtype=torch.int8, device=device)
-        act_scale = torch.empty(T, dtype=torch.float32, device=device)
-        xp = torch.empty((T, k), dtype=torch.float32, device=device)
-        wp = torch.empty((out, k), dtype=torch.float32, device=device)
+        # one allocation for the column maxima, codes, scales and side operands
+        sizes = (4 * ((T + 1023) // 1024) * inn, T * inn, 4 * T, 4 * T * k, 4 * out * k)
+        at = [0]
+        for size in sizes:
+            at.append((at[-1] + size + 255) // 256 * 256)
+        ws = torch.empty(at[-1], dtype=torch.uint8, device=device)
+        colws, q_x, act_scale, xp, wp = (nat.ptr(ws) + o for o in at[:-1])
         nat.call("qs_w8a8_protect_quant", nat.ptr(x2), xdt, inn, T, inn, k, nat.ptr(q_w), nat.ptr(sc_w), out,
-                 nat.ptr(colws), nat.ptr(q_x), nat.ptr(act_scale), nat.ptr(xp), nat.ptr(wp), None, None, stream)
-        nat.call("qs_w8a8_gemm", nat.ptr(q_x), nat.ptr(act_scale), nat.ptr(q_w), nat.ptr(sc_w), nat.ptr(xp),
-                 nat.ptr(wp), k, nat.ptr(y), nat.dtype_code(out_dtype), T, out, inn, stream)
-        return y.reshape(*x.shape[:-1], out)
+                 colws, q_x, act_scale, xp, wp, None, None, stream)
+        nat.call("qs_w8a8_gemm", q_x, act_scale, nat.ptr(q_w), nat.ptr(sc_w), xp, wp, k, nat.ptr(y),
+                 nat.dtype_code(out_dtype), T, out, inn, stream)
+        return y if x.ndim == 2 else y.reshape(*x.shape[:-1], out)
     if protect_idx is None and protect_k > 0:
         k = min(int(protect_k), inn)
         colmax = torch.empty(inn, dtype=torch.float32, device=device)
