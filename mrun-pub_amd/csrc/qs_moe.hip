@@ -502,6 +502,82 @@ __device__ __forceinline__ GroupMeta group_meta(const int32_t* counts, const int
   return GroupMeta{c, st, slots ? sv : g};
 }
 
+// Work item of a streaming workgroup: a group with rows and one of its rb row blocks.
+struct WorkItem {
+  GroupMeta gm;
+  int bx;
+};
+constexpr int kPickGroups = 512;  // groups whose counts a wave holds in registers
+
+// Workgroup i runs on XCD i % 8.  The row blocks of one group share its staged routed rows, so
+// the group-major list of row blocks is dealt out XCD by XCD and one L2 serves the repeats.
+//
+// Not `sparse` (nearly every group has rows): a grid of (rb, G), its first 8 * floor(total / 8)
+// workgroups XCD-major, the remainder in its own place (a bijection on [0, total)); a workgroup
+// of an empty group ends.
+//
+// `sparse`: 8 * ceil(rb * G / 8) workgroups over the list of the groups that have rows, of which
+// every XCD takes an equal run.  (With the empty groups dealt out too, each XCD has the rows of
+// its own 16 of 128 experts: at 13 tokens, 72 active experts on average, the fullest XCD had a
+// third more than the mean and the others waited: gate/up 64 -> 49 us.)  Each wave reads all
+// counts at once and finds its group by ballots.
+// false: nothing to do.
+__device__ __forceinline__ bool pick_item(const int32_t* counts, const int32_t* starts, const int32_t* slots, int G,
+                                          int rb, bool sparse, WorkItem& it) {
+  const int lane = (int)threadIdx.x & 63;
+  if (!sparse) {
+    const int total = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
+    const int per_xcd = total / 8;
+    const int logical = lin < 8 * per_xcd ? (lin % 8) * per_xcd + lin / 8 : lin;
+    const int g = logical / gridDim.x;
+    it.bx = logical - g * gridDim.x;
+    it.gm = group_meta(counts, starts, slots, g);
+    return it.gm.count > 0;
+  }
+  const int lin = (int)blockIdx.x, xcd = lin & 7, idx = lin >> 3;
+  constexpr int R = kPickGroups / 64;
+  const int32_t* sp = slots ? slots : starts;
+  int c[R], st[R], sl[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    c[i] = st[i] = sl[i] = 0;
+    if (64 * i < G) {
+      const int g = min(64 * i + lane, G - 1);
+      c[i] = counts[g];
+      st[i] = starts[g];
+      sl[i] = sp[g];
+    }
+  }
+  unsigned long long has[R];
+  int n = 0;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    has[i] = __ballot(64 * i + lane < G && c[i] > 0);
+    n += __popcll(has[i]);
+  }
+  const int items = n * rb, per = (items + 7) >> 3;
+  const int item = xcd * per + idx;
+  if (idx >= per || item >= items) return false;
+  int a = item / rb;  // the a-th group with rows
+  it.bx = item - a * rb;
+  it.gm = GroupMeta{0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int here = __popcll(has[i]);
+    if (a >= 0 && a < here) {
+      const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(has[i] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)has[i], 0));
+      const unsigned long long at = __ballot((has[i] >> lane & 1) && rank == a);
+      const int l = __ffsll((long long)at) - 1;
+      it.gm.count = __builtin_amdgcn_readlane(c[i], l);
+      it.gm.start = __builtin_amdgcn_readlane(st[i], l);
+      const int v = __builtin_amdgcn_readlane(sl[i], l);
+      it.gm.slot = slots ? v : 64 * i + l;
+    }
+    a -= here;  // negative once the group is found
+  }
+  return true;
+}
+
 struct MoeGemmParams {
   const int8_t* a;       // [A, K] routed rows, expert-major
   const float* as;       // [A]
@@ -518,6 +594,8 @@ struct MoeGemmParams {
   int out_dtype;
   const int64_t* row_ids;  // k_moe_stream, nullable: queue row r reads a / as at row_ids[r]
   int64_t src_rows;        // rows of a and as when row_ids is given
+  int G, rb;               // k_moe_stream: groups, and row blocks per group
+  bool sparse;             // k_moe_stream: groups without rows are expected
 };
 
 __device__ __forceinline__ float silu_f(float g) { return g * (1.0f / (1.0f + expf(-g))); }
@@ -668,17 +746,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_moe_stream(MoeGemmParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, q = lane >> 4;
-  // Workgroup i runs on XCD i % 8.  The row blocks of one group share its staged routed
-  // rows, so consecutive logical indices (group-major) go to one XCD and its L2 serves
-  // the repeats: the first 8 * floor(total / 8) workgroups are dealt out XCD-major, the
-  // remainder keeps its index (a bijection on [0, total)).
-  const int total = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
-  const int per_xcd = total / 8;
-  const int logical = lin < 8 * per_xcd ? (lin % 8) * per_xcd + lin / 8 : lin;
-  const int g = logical / gridDim.x, bx = logical - g * gridDim.x;
-  const GroupMeta gm = group_meta(p.counts, p.starts, p.slots, g);
+  WorkItem it;
+  if (!pick_item(p.counts, p.starts, p.slots, p.G, p.rb, p.sparse, it)) return;
+  const GroupMeta gm = it.gm;
+  const int bx = it.bx;
   const int count = gm.count;
-  if (count == 0) return;
   const int start = gm.start;
   const int slot = gm.slot;
   const int K = p.K, C = K / CB;
@@ -852,6 +924,8 @@ struct MoeW16Params {
   int N, K, KPH;
   void* out;
   int out_dtype;
+  int G, rb;  // groups, and row blocks per group
+  bool sparse;  // groups without rows are expected
 };
 
 template <int P, int NB, int MT, int W, int WAVES, int PAIR>
@@ -866,13 +940,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_moe_stream_w16(MoeW16Params p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, q = lane >> 4;
-  const int total = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
-  const int per_xcd = total / 8;
-  const int logical = lin < 8 * per_xcd ? (lin % 8) * per_xcd + lin / 8 : lin;
-  const int g = logical / gridDim.x, bx = logical - g * gridDim.x;
-  const GroupMeta gm = group_meta(p.counts, p.starts, p.slots, g);
+  WorkItem it;
+  if (!pick_item(p.counts, p.starts, p.slots, p.G, p.rb, p.sparse, it)) return;
+  const GroupMeta gm = it.gm;
+  const int bx = it.bx;
   const int count = gm.count;
-  if (count == 0) return;
   const int start = gm.start;
   const int slot = gm.slot;
   const int K = p.K, C = K / CB, KPH = p.KPH, CPH = KPH / CB;
@@ -1229,6 +1301,20 @@ extern "C" int qs_moe_gather_quant(const void* source, int src_dtype, int64_t ld
 }
 
 namespace {
+// pick_item's list of the groups with rows: for fewer than `rows` routed rows per group on
+// average.  3 for w8a16 pages (an even routing leaves 5% of the groups empty there), 2 for int8
+// (14%), whose shorter blocks notice the list's longer start sooner.  The layer of 128 experts,
+// top-8, by tokens, one mapping then the other: w8a16 1: 58 -> 39 us, 13: 101 -> 88,
+// 32: 127 -> 121, 45: 132 -> 126, 64: equal; int8 1: 50 -> 33, 13: 99 -> 89, 32: equal,
+// 45: 124 -> 126.
+bool moe_sparse(int64_t max_rows, int G, int rows) {
+  return G <= kPickGroups && max_rows > 0 && max_rows < (int64_t)rows * G;
+}
+
+dim3 moe_stream_grid(bool sparse, int rb, int G) {
+  return sparse ? dim3((unsigned)(cdiv((int64_t)rb * G, 8) * 8)) : dim3((unsigned)rb, (unsigned)G);
+}
+
 constexpr int kMoeTilesPerBlock = 1;  // 16-row tiles per workgroup, streamed back to back
 constexpr size_t kMoeStreamLds = 144 * 1024;  // staged routed rows of k_moe_stream
 
@@ -1255,14 +1341,16 @@ size_t moe_stream_lds(int MT, int64_t K) {
 // 8 waves for two and 12 for four; two 128-byte chunks in flight.  Plain products keep 128 bytes
 // of each weight row in flight for NB >= 2 tiles per wave, 256 for one.
 template <int P, int NB, int MT, int PAIR, int WAVES_SET = 0>
-void launch_moe_stream_mt(const MoeGemmParams& p, int G, hipStream_t s) {
+void launch_moe_stream_mt(MoeGemmParams p, int G, hipStream_t s) {
   // SwiGLU with 64-row passes: 12 waves (N = 768: four workgroups per expert, two full
   // rounds of the CUs at 128 experts; T = 512 gate/up 85.3 -> 82.6 us against 8 waves)
   constexpr int WAVES = WAVES_SET ? WAVES_SET : (P == 2 ? (MT == 1 ? 4 : (MT == 4 ? 12 : 8)) : 4);
   constexpr int WP = P == 2 ? 2 : (NB >= 2 ? 1 : 2);  // 128-byte chunks in flight
   constexpr int W = PAIR ? WP : 2 * WP;
   constexpr int RW = MoeStreamCfg<P, NB>::RW;
-  const dim3 grid((unsigned)cdiv(p.N, RW * WAVES), (unsigned)G), block(WAVES * 64);
+  p.G = G;
+  p.rb = (int)cdiv(p.N, RW * WAVES);
+  const dim3 grid = moe_stream_grid(p.sparse, p.rb, G), block(WAVES * 64);
   hipLaunchKernelGGL((k_moe_stream<P, NB, MT, W, WAVES, PAIR>), grid, block, moe_stream_lds(MT, p.K), s, p);
 }
 
@@ -1303,7 +1391,9 @@ void launch_moe_w16_mt(MoeW16Params p, int G, size_t cap, hipStream_t s) {
   constexpr int RW = MoeStreamCfg<P, NB>::RW;
   p.KPH = moe_w16_phase(MT, p.K, PAIR ? 128 : 64, W, cap);
   const size_t lds = (size_t)16 * MT * (size_t)(2 * p.KPH + 16 + 8);  // staged rows + their ids
-  const dim3 grid((unsigned)cdiv(p.N, RW * WAVES), (unsigned)G), block(WAVES * 64);
+  p.G = G;
+  p.rb = (int)cdiv(p.N, RW * WAVES);
+  const dim3 grid = moe_stream_grid(p.sparse, p.rb, G), block(WAVES * 64);
   hipLaunchKernelGGL((k_moe_stream_w16<P, NB, MT, W, WAVES, PAIR>), grid, block, lds, s, p);
 }
 
@@ -1354,7 +1444,7 @@ extern "C" int qs_moe_grouped_gemm_w8a16(const void* a, const int64_t* row_ids, 
   if (max_rows < 0) return fail(QS_ERR_INVALID, "moe_grouped_gemm_w8a16: max_rows must be >= 0");
   if (src_rows > (int64_t)1 << 40) return fail(QS_ERR_LIMIT, "moe_grouped_gemm_w8a16: src_rows too large");
   MoeW16Params p{static_cast<const uint16_t*>(a), row_ids, src_rows, w, w_stride, w_scale, ws_stride,
-                 starts, counts, slots, (int)N, (int)K, 0, out, out_dtype};
+                 starts, counts, slots, (int)N, (int)K, 0, out, out_dtype, 0, 0, moe_sparse(max_rows, G, 3)};
   hipStream_t s = static_cast<hipStream_t>(stream);
   // row tiles sized for twice the mean rows per group, as the int8 stream
   const int64_t mean = max_rows > 0 ? cdiv(max_rows, G) : 16;
@@ -1380,7 +1470,7 @@ int grouped_gemm_i8(const int8_t* a, const float* a_scale, const int64_t* row_id
   if (max_rows < 0) return fail(QS_ERR_INVALID, "moe_grouped_gemm: max_rows must be >= 0");
   if (src_rows < 0) return fail(QS_ERR_INVALID, "moe_grouped_gemm: src_rows must be >= 0");
   MoeGemmParams p{a, a_scale, w, w_stride, w_scale, ws_stride, starts, counts, slots, (int)N, (int)K, out, out_dtype,
-                  row_ids, src_rows};
+                  row_ids, src_rows, 0, 0, moe_sparse(max_rows, G, 2)};
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Streaming kernel: row tiles sized for twice the mean rows per group (max_rows / G),
   // so that most groups take one pass over their weights; 0 = unknown -> 2 tiles.

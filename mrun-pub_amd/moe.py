@@ -283,7 +283,7 @@ def grouped_int8_mm(
     as up and returns ``bf16(silu(gate) * up)`` of width ``N/2``.  ``max_rows`` bounds
     every group's row count as in the reference's grouped kernels
     (qwen3_moe_cuda.py:2257-2310); it defaults to the routed row count, as its callers
-    pass (:2747), and only sizes the kernel's row tile.
+    pass (:2747), and only chooses the kernel's row tile and split over the chip.
     """
     G, n_w, K = _grouped_contract(rows_q, weights, weight_scales, starts, counts, group_slots)
     device = nat.require_device(rows_q, row_scales, weights, weight_scales, starts, counts, group_slots, row_ids)

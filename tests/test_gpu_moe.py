@@ -472,3 +472,38 @@ def test_moe_layer_graph_replays_equal_eager(dev, w8a16):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), f"replay {rep}"
+
+
+# groups: less than one XCD's share, edges of the 64 counts a wave reads at once, and the last
+# size that is listed and the first that is not; rows: one group, a few, most groups
+@pytest.mark.parametrize("w16", [False, True])
+@pytest.mark.parametrize("G,rows", [(1, 1), (5, 3), (63, 1), (64, 9), (65, 40), (130, 128), (512, 300), (513, 300)])
+def test_grouped_gemm_few_active_groups(dev, G, rows, w16):
+    """Launches that list the groups with rows equal those that deal out all groups, and the
+    oracle, with direct and permuted weight slots."""
+    rng = np.random.default_rng(G + rows)
+    K, N = 128, 160
+    w = rng.integers(-127, 128, size=(G, N, K), dtype=np.int8)
+    ws = rng.uniform(0.01, 0.1, size=(G, N)).astype(np.float32)
+    counts = np.bincount(rng.integers(0, G, size=rows), minlength=G).astype(np.int32)
+    starts = (np.cumsum(counts) - counts).astype(np.int32)
+    perm = rng.permutation(G)
+    slots = _t(np.argsort(perm).astype(np.int32), dev)
+    wt, wst, wp, wsp = (_t(v, dev) for v in (w, ws, w[perm], ws[perm]))
+    st, ct = _t(starts, dev), _t(counts, dev)
+    for swiglu in (False, True):
+        if w16:
+            x = _w16_rows(rng, rows, K)
+            run = lambda wv, sv, **kw: _moe().grouped_w8a16_mm(  # noqa: E731
+                _t(x, dev, torch.bfloat16), wv, sv, st, ct, swiglu=swiglu, **kw)[0]
+            ref = om.grouped_w8a16_mm(x, w, ws, starts, counts, swiglu=swiglu)
+        else:
+            a = rng.integers(-127, 128, size=(rows, K), dtype=np.int8)
+            asc = rng.uniform(0.01, 0.1, size=rows).astype(np.float32)
+            run = lambda wv, sv, **kw: _moe().grouped_int8_mm(  # noqa: E731
+                _t(a, dev), _t(asc, dev), wv, sv, st, ct, swiglu=swiglu, **kw)[0]
+            ref = om.grouped_int8_mm(a, asc, w, ws, starts, counts, swiglu=swiglu)
+        listed = run(wt, wst)
+        assert oq.rel_l2(listed.float().cpu().numpy(), ref) <= 1e-3
+        assert torch.equal(run(wp, wsp, group_slots=slots), listed)
+        assert torch.equal(run(wt, wst, max_rows=0), listed)  # 0: all groups dealt out
