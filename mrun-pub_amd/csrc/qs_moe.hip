@@ -521,11 +521,13 @@ constexpr int kPickGroups = 512;  // groups whose counts a wave holds in registe
 // its own 16 of 128 experts: at 13 tokens, 72 active experts on average, the fullest XCD had a
 // third more than the mean and the others waited: gate/up 64 -> 49 us.)  Each wave reads all
 // counts at once and finds its group by ballots.
+// Only kernels of one row tile have it: `sparse` launches are of few rows per group.
 // false: nothing to do.
+template <int MT>
 __device__ __forceinline__ bool pick_item(const int32_t* counts, const int32_t* starts, const int32_t* slots, int G,
                                           int rb, bool sparse, WorkItem& it) {
   const int lane = (int)threadIdx.x & 63;
-  if (!sparse) {
+  if (MT > 1 || !sparse) {
     const int total = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
     const int per_xcd = total / 8;
     const int logical = lin < 8 * per_xcd ? (lin % 8) * per_xcd + lin / 8 : lin;
@@ -747,7 +749,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_moe_stream(MoeGemmParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, q = lane >> 4;
   WorkItem it;
-  if (!pick_item(p.counts, p.starts, p.slots, p.G, p.rb, p.sparse, it)) return;
+  if (!pick_item<MT>(p.counts, p.starts, p.slots, p.G, p.rb, p.sparse, it)) return;
   const GroupMeta gm = it.gm;
   const int bx = it.bx;
   const int count = gm.count;
@@ -941,7 +943,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_moe_stream_w16(MoeW16Params p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, q = lane >> 4;
   WorkItem it;
-  if (!pick_item(p.counts, p.starts, p.slots, p.G, p.rb, p.sparse, it)) return;
+  if (!pick_item<MT>(p.counts, p.starts, p.slots, p.G, p.rb, p.sparse, it)) return;
   const GroupMeta gm = it.gm;
   const int bx = it.bx;
   const int count = gm.count;
@@ -1350,6 +1352,7 @@ void launch_moe_stream_mt(MoeGemmParams p, int G, hipStream_t s) {
   constexpr int RW = MoeStreamCfg<P, NB>::RW;
   p.G = G;
   p.rb = (int)cdiv(p.N, RW * WAVES);
+  p.sparse = p.sparse && MT == 1;
   const dim3 grid = moe_stream_grid(p.sparse, p.rb, G), block(WAVES * 64);
   hipLaunchKernelGGL((k_moe_stream<P, NB, MT, W, WAVES, PAIR>), grid, block, moe_stream_lds(MT, p.K), s, p);
 }
@@ -1393,6 +1396,7 @@ void launch_moe_w16_mt(MoeW16Params p, int G, size_t cap, hipStream_t s) {
   const size_t lds = (size_t)16 * MT * (size_t)(2 * p.KPH + 16 + 8);  // staged rows + their ids
   p.G = G;
   p.rb = (int)cdiv(p.N, RW * WAVES);
+  p.sparse = p.sparse && MT == 1;
   const dim3 grid = moe_stream_grid(p.sparse, p.rb, G), block(WAVES * 64);
   hipLaunchKernelGGL((k_moe_stream_w16<P, NB, MT, W, WAVES, PAIR>), grid, block, lds, s, p);
 }
