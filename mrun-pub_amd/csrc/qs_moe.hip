@@ -46,7 +46,10 @@ __device__ __forceinline__ float ld(const void* p, int64_t i) {
 }
 
 // E <= 64 * J logits per wave (J per lane), k <= 16.  Rank r is kept by lane r (no
-// dynamically indexed arrays, which would live in scratch memory).
+// dynamically indexed arrays, which would live in scratch memory).  A chain of k dependent
+// selections bounds it: each takes the maximum by register lane moves and finds its lowest
+// index by ballots (128 logits, top-8, 13 and 777 tokens: 7.1 -> 4.4 us against a butterfly of
+// value and index through LDS permutes).
 template <int XT, int J>
 __global__ __launch_bounds__(256) void k_moe_router(const void* __restrict__ logits, int T, int E,
                                                     int k, int norm, int64_t* __restrict__ idx,
@@ -72,29 +75,21 @@ __global__ __launch_bounds__(256) void k_moe_router(const void* __restrict__ log
   }
   sum = wave_sum(sum);
 #pragma unroll
-  for (int j = 0; j < J; ++j) v[j] = v[j] / sum;
+  for (int j = 0; j < J; ++j) v[j] = lane + 64 * j < E ? v[j] / sum : -2.f;  // -2: never taken
   float mine = 0.f;  // lane r: the weight of rank r
   int mine_idx = 0;
   float tot = 0.f;   // fp32 sum of the kept weights in rank order
   for (int r = 0; r < k; ++r) {
     float best = -1.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) best = fmaxf(best, v[j]);
+    best = wave_max(best);
+    // lowest e that holds it (e = lane + 64 j); none (NaN logits): 0x7fffffff, weight -1
     int bi = 0x7fffffff;
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int e = lane + 64 * j;
-      if (e < E && (v[j] > best || (v[j] == best && e < bi))) {
-        best = v[j];
-        bi = e;
-      }
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      const float ob = __shfl_xor(best, off, 64);
-      const int oi = __shfl_xor(bi, off, 64);
-      if (ob > best || (ob == best && oi < bi)) {
-        best = ob;
-        bi = oi;
-      }
+    for (int j = J - 1; j >= 0; --j) {
+      const uint64_t at = __ballot(v[j] == best);
+      bi = at ? 64 * j + __ffsll((long long)at) - 1 : bi;
     }
     if (lane == r) {
       mine = best;

@@ -507,3 +507,23 @@ def test_grouped_gemm_few_active_groups(dev, G, rows, w16):
         assert oq.rel_l2(listed.float().cpu().numpy(), ref) <= 1e-3
         assert torch.equal(run(wp, wsp, group_slots=slots), listed)
         assert torch.equal(run(wt, wst, max_rows=0), listed)  # 0: all groups dealt out
+
+
+# expert counts around the 64 logits a wave's register holds, and the 16-register form
+@pytest.mark.parametrize("E", [3, 63, 64, 65, 128, 300, 1000])
+def test_router_ties_and_nan(dev, E):
+    """Equal weights are taken in index order; a NaN row yields no index (and no fault)."""
+    rng = np.random.default_rng(E)
+    k = min(16, E)
+    logits = rng.integers(0, 3, size=(9, E)).astype(np.float32)  # three levels: ties in every row
+    logits[4] = 0.5
+    logits[7, E // 2] = np.nan
+    w, idx = _moe().route_topk(_t(logits, dev), k, norm_topk=False, out_dtype=torch.float32)
+    ok = np.arange(9) != 7
+    want = np.argsort(-logits[ok], axis=1, kind="stable")[:, :k]
+    assert np.array_equal(idx.cpu().numpy()[ok], want)
+    p = np.exp(logits[ok].astype(np.float64))
+    p /= p.sum(axis=1, keepdims=True)
+    # exp, at most 16 + 6 roundings of the sum, and the division: 25 * 2^-24 relative
+    np.testing.assert_allclose(w.cpu().numpy()[ok], np.take_along_axis(p, want, 1), rtol=1.5e-6)
+    assert (idx.cpu().numpy()[7] == 0x7FFFFFFF).all() and (w.cpu().numpy()[7] == -1).all()
