@@ -1308,6 +1308,10 @@ bool moe_sparse(int64_t max_rows, int G, int rows) {
   return G <= kPickGroups && max_rows > 0 && max_rows < (int64_t)rows * G;
 }
 
+// A sparse launch whose blocks of 64 output rows, at most one group per routed row, are no more
+// than the chip's 256 CUs.
+bool moe_few(bool sparse, int64_t max_rows, int64_t N) { return sparse && max_rows * cdiv(N, 64) <= 256; }
+
 dim3 moe_stream_grid(bool sparse, int rb, int G) {
   return sparse ? dim3((unsigned)(cdiv((int64_t)rb * G, 8) * 8)) : dim3((unsigned)rb, (unsigned)G);
 }
@@ -1381,10 +1385,15 @@ int moe_w16_phase(int MT, int64_t K, int CB, int W, size_t cap) {
 // staged slice at 72 KB so that two or three workgroups share a CU (T = 512 down
 // 74 -> 51 us); shorter passes use 8 waves of at most 2 tiles (T = 64 down 41 -> 36 us).
 // The dequantization costs 2.5 VALU operations per code, so the stream needs more waves
-// per SIMD than the int8 one to keep its loads in flight.
-template <int P, int NB, int MT, int PAIR, int WAVES>
+// per SIMD than the int8 one to keep its loads in flight.  Sparse launches have fewer blocks than
+// the chip holds at once, and the CU with one block more than the others sets the time: plain
+// products halve the block (us at 1, 13, 20, 31 tokens: 11.0, 30.0, 39.6, 41.3 -> 9.3, 25.3,
+// 35.4, 39.1).  Launches of few blocks (moe_few) take the smaller ones with more chunks in
+// flight: gate/up at 1 and 2 tokens 21.3 -> 14.5 and 22.2 -> 16.1 (at 4 tokens 23.1 -> 24.6, at
+// 13 47 -> 50), down at 1 token 11.0 -> 7.5.
+template <int P, int NB, int MT, int PAIR, int WAVES, int WP_SET = 0>
 void launch_moe_w16_mt(MoeW16Params p, int G, size_t cap, hipStream_t s) {
-  constexpr int WP = P == 2 ? 2 : (NB >= 2 ? 1 : 2);  // w16 chunks in flight
+  constexpr int WP = WP_SET ? WP_SET : (P == 2 ? 2 : (NB >= 2 ? 1 : 2));  // w16 chunks in flight
   constexpr int W = PAIR ? WP : 2 * WP;
   constexpr int RW = MoeStreamCfg<P, NB>::RW;
   p.KPH = moe_w16_phase(MT, p.K, PAIR ? 128 : 64, W, cap);
@@ -1396,16 +1405,17 @@ void launch_moe_w16_mt(MoeW16Params p, int G, size_t cap, hipStream_t s) {
   hipLaunchKernelGGL((k_moe_stream_w16<P, NB, MT, W, WAVES, PAIR>), grid, block, lds, s, p);
 }
 
-template <int P, int NB, int MT, int WAVES>
+template <int P, int NB, int MT, int WAVES, int WP_SET = 0>
 void launch_moe_w16_pair(const MoeW16Params& p, int G, size_t cap, hipStream_t s) {
-  if (p.K % 128 == 0) launch_moe_w16_mt<P, NB, MT, 1, WAVES>(p, G, cap, s);
-  else launch_moe_w16_mt<P, NB, MT, 0, WAVES>(p, G, cap, s);
+  if (p.K % 128 == 0) launch_moe_w16_mt<P, NB, MT, 1, WAVES, WP_SET>(p, G, cap, s);
+  else launch_moe_w16_mt<P, NB, MT, 0, WAVES, WP_SET>(p, G, cap, s);
 }
 
-void launch_moe_w16(const MoeW16Params& p, int G, int MT, bool swiglu, hipStream_t s) {
+void launch_moe_w16(const MoeW16Params& p, int G, int MT, bool swiglu, bool few, hipStream_t s) {
   const int64_t K = p.K;
   if (swiglu) {
-    if (MT == 4) launch_moe_w16_pair<2, 2, 4, 12>(p, G, kMoeStreamLds, s);  // 102.1 -> 91.2 us at T = 512 (8 waves)
+    if (few) launch_moe_w16_pair<2, 2, 1, 4, 4>(p, G, kMoeStreamLds, s);
+    else if (MT == 4) launch_moe_w16_pair<2, 2, 4, 12>(p, G, kMoeStreamLds, s);  // 102.1 -> 91.2 us at T = 512 (8 waves)
     else if (MT == 2) launch_moe_w16_pair<2, 2, 2, 8>(p, G, kMoeStreamLds, s);
     else launch_moe_w16_pair<2, 2, 1, 8>(p, G, kMoeStreamLds, s);  // T = 64 layer 128.8 -> 125.3 us (4 waves)
   } else if (MT == 4) {
@@ -1416,8 +1426,11 @@ void launch_moe_w16(const MoeW16Params& p, int G, int MT, bool swiglu, hipStream
   } else if (MT == 2) {
     if (K <= 2048) launch_moe_w16_pair<1, 2, 2, 8>(p, G, kMoeStreamLds, s);
     else launch_moe_w16_pair<1, 1, 2, 8>(p, G, kMoeStreamLds, s);
+  } else if (few) {
+    launch_moe_w16_pair<1, 1, 1, 4>(p, G, kMoeStreamLds, s);
   } else {
-    if (K <= 2048) launch_moe_w16_pair<1, 2, 1, 8>(p, G, kMoeStreamLds, s);
+    if (K <= 2048 && p.sparse) launch_moe_w16_pair<1, 2, 1, 4>(p, G, kMoeStreamLds, s);
+    else if (K <= 2048) launch_moe_w16_pair<1, 2, 1, 8>(p, G, kMoeStreamLds, s);
     else launch_moe_w16_pair<1, 1, 1, 8>(p, G, kMoeStreamLds, s);
   }
 }
@@ -1448,7 +1461,7 @@ extern "C" int qs_moe_grouped_gemm_w8a16(const void* a, const int64_t* row_ids, 
   // row tiles sized for twice the mean rows per group, as the int8 stream
   const int64_t mean = max_rows > 0 ? cdiv(max_rows, G) : 16;
   const int MT = 2 * mean <= 16 ? 1 : (2 * mean <= 32 ? 2 : 4);
-  launch_moe_w16(p, G, MT, swiglu != 0, s);
+  launch_moe_w16(p, G, MT, swiglu != 0, moe_few(p.sparse, max_rows, N), s);
   return hip_check(hipGetLastError(), "k_moe_stream_w16 launch");
 }
 
@@ -1480,13 +1493,19 @@ int grouped_gemm_i8(const int8_t* a, const float* a_scale, const int64_t* row_id
   // 128-byte chunk loads the stream also beats it on short groups: T = 64 down 50 -> 42 us).
   if (moe_stream_lds(MT, K)) {
     // plain: row tiles per wave so that a wave streams about 48 KB or more
-    if (swiglu) launch_moe_stream<2, 2>(p, G, MT, s);
+    if (swiglu && moe_few(p.sparse, max_rows, N)) {
+      // blocks of two waves: gate/up at 1 token 12.2 -> 8.7 us, at 2 level
+      if (K % 128 == 0) launch_moe_stream_mt<2, 2, 1, 1, 2>(p, G, s);
+      else launch_moe_stream_mt<2, 2, 1, 0, 2>(p, G, s);
+    } else if (swiglu) launch_moe_stream<2, 2>(p, G, MT, s);
     else if (K <= 1024 && MT == 4) {
       // 64-row passes of short rows (T = 512 down): 8 waves of two tiles (43.0 -> 40.0 us;
       // shorter passes keep 4 waves of four tiles: T = 64 down 34.2 against 35.4)
       if (K % 128 == 0) launch_moe_stream_mt<1, 2, 4, 1, 8>(p, G, s);
       else launch_moe_stream_mt<1, 2, 4, 0, 8>(p, G, s);
-    } else if (K <= 1024) launch_moe_stream<1, 4>(p, G, MT, s);
+    } else if (K <= 1024 && !p.sparse) launch_moe_stream<1, 4>(p, G, MT, s);
+    // sparse, K <= 1024: two tiles per wave, so that more and smaller blocks spread more evenly
+    // (T = 1, 13, 20, 31 down: 10.8, 28.6, 37.5, 38.5 -> 7.8, 25.9, 34.4, 38.8 us)
     else if (K <= 2048) launch_moe_stream<1, 2>(p, G, MT, s);
     else launch_moe_stream<1, 1>(p, G, MT, s);
     return hip_check(hipGetLastError(), "k_moe_stream launch");

@@ -475,14 +475,17 @@ def test_moe_layer_graph_replays_equal_eager(dev, w8a16):
 
 
 # groups: less than one XCD's share, edges of the 64 counts a wave reads at once, and the last
-# size that is listed and the first that is not; rows: one group, a few, most groups
+# size that is listed and the first that is not; rows: one group, a few (the smaller blocks
+# end at 85 rows for N = 160), most groups; K: one 64-code chunk, odd and even numbers of them,
+# and two staged phases of weight-only rows (6208, 6272)
 @pytest.mark.parametrize("w16", [False, True])
-@pytest.mark.parametrize("G,rows", [(1, 1), (5, 3), (63, 1), (64, 9), (65, 40), (130, 128), (512, 300), (513, 300)])
-def test_grouped_gemm_few_active_groups(dev, G, rows, w16):
+@pytest.mark.parametrize("G,rows,K", [(1, 1, 64), (5, 3, 6208), (63, 1, 6272), (64, 9, 192), (65, 40, 1152), (65, 85, 128),
+                                      (65, 86, 128), (130, 128, 128), (512, 300, 128), (513, 300, 128)])
+def test_grouped_gemm_few_active_groups(dev, G, rows, K, w16):
     """Launches that list the groups with rows equal those that deal out all groups, and the
     oracle, with direct and permuted weight slots."""
     rng = np.random.default_rng(G + rows)
-    K, N = 128, 160
+    N = 160
     w = rng.integers(-127, 128, size=(G, N, K), dtype=np.int8)
     ws = rng.uniform(0.01, 0.1, size=(G, N)).astype(np.float32)
     counts = np.bincount(rng.integers(0, G, size=rows), minlength=G).astype(np.int32)
