@@ -112,24 +112,9 @@ __device__ __forceinline__ void deq16_f16(i32x4 w, float s, f16x8& lo, f16x8& hi
 
 // Full-wave sum with a fixed butterfly order (deterministic, identical for every
 // call with the same operand).
-// v's exchange partner at distance 8, 4, 2 or 1 once the distances above it are done, all 64
-// lanes active.  After the exchange at distance 8 (a rotation of the 16-lane row by 8) lanes
-// agree modulo 8, so a rotation by 4 has the operand of the exchange at distance 4.
-template <int DIST>
-__device__ __forceinline__ float dpp_partner(float v) {
-  constexpr int ctrl = DIST == 8 ? 0x128 : DIST == 4 ? 0x124 : DIST == 2 ? 0x4E : 0xB1;  // row_ror:8, :4, quad_perm
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xf, 0xf, false));
-}
-
-// Butterfly sum, distances 32, 16, 8, 4, 2, 1; every lane gets it.  The last four are register
-// lane moves (an LDS permute costs a dependent step about 100 cycles).
 __device__ __forceinline__ float wave_sum(float v) {
-  v += __shfl_xor(v, 32, kWave);
-  v += __shfl_xor(v, 16, kWave);
-  v += dpp_partner<8>(v);
-  v += dpp_partner<4>(v);
-  v += dpp_partner<2>(v);
-  v += dpp_partner<1>(v);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, kWave);
   return v;
 }
 

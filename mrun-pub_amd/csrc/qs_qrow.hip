@@ -1286,10 +1286,9 @@ __global__ __launch_bounds__(512) void k_gemv_top2_xg(QrowParams p, int rows, in
 // across tile boundaries.  Dequantized weights are the A operand, so lane l holds the logits
 // of weight rows 4 (l >> 4) + 0..3 for activation row l & 15 and keeps that row's running
 // first and second.  Four accumulators per tile keep the fp32 chains as short as the VALU
-// kernel's.  Eleven bf16 rows: 269 -> 67 us with the rerank (this
-// launch 55); fp32 rows run 16x16x4 MFMAs,
-// whose rate bounds them (eleven rows of
-// 151,936 x 1536 without the rerank: 315 -> 117 us; bf16 292 -> 61).
+// kernel's.  Eleven bf16 rows: 269 -> 67 us with the rerank (this launch 55); fp32 rows run
+// 16x16x4 MFMAs, whose rate bounds them (eleven rows of 151,936 x 1536 without the rerank:
+// 315 -> 117 us; bf16 292 -> 61).
 template <int XT, int W>
 __global__ __launch_bounds__(512) void k_head_top2(QrowParams p, int rows, int start_row, float* part_v,
                                                    int* part_i) {
@@ -2149,8 +2148,9 @@ int top2_validate(const void* x, int x_dtype, int64_t ldx, const int8_t* codes, 
 // whose 16-row tile fits LDS.
 bool head_tile_ok(const QrowParams& p, int x_dtype, int64_t M) {
   const int es = x_dtype == QS_F32 ? 4 : 2;
-  return M >= (x_dtype == QS_F32 ? 5 : 3) && p.K % 128 == 0 && p.K >= 512 && (int64_t)16 * p.K * es <= 144 * 1024 && p.ldx * es % 16 == 0 &&
-         aligned(p.x, 16) && aligned(p.lin[0].codes, 16);
+  return M >= (x_dtype == QS_F32 ? 5 : 3) && p.K % 128 == 0 && p.K >= 512 &&
+         (int64_t)16 * p.K * es <= 144 * 1024 && p.ldx * es % 16 == 0 && aligned(p.x, 16) &&
+         aligned(p.lin[0].codes, 16);
 }
 
 // Workgroups of k_head_top2 (8 waves of 16-row tiles): as many as are resident, two per CU
