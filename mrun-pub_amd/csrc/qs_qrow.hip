@@ -1649,11 +1649,13 @@ bool stream_fits(const QrowParams& q) {
 // LDS bytes for the activations of the streaming kernel, 0 when they are read from
 // L2: a copy per workgroup pays off while it is small next to the workgroup's weights --
 // up to 25 KB (M <= 8 rows of a 1536-wide layer), or up to 144 KB when the launch has
-// at most one workgroup per CU anyway (few, long tiles such as 1536 x 8960).
-size_t stream_xl_bytes(const QrowParams& q, int blocks) {
+// at most one workgroup per CU anyway (few, long tiles such as 1536 x 8960) and they fit the
+// CU's 160 KB beside the workgroup's own `fixed` bytes (its slice sums: 32 KB for two
+// activation tiles of 8 two-plane or 16 one-plane slices, 16 KB or less otherwise).
+size_t stream_xl_bytes(const QrowParams& q, int blocks, size_t fixed) {
   const size_t b = (size_t)q.M * (size_t)(2 * q.K + 16);
   if (b <= 25 * 1024) return b;
-  if (blocks <= 256 && b <= 144 * 1024) return b;
+  if (blocks <= 256 && b <= 144 * 1024 && b + fixed <= 160 * 1024) return b;
   return 0;
 }
 
@@ -1662,7 +1664,7 @@ size_t stream_xl_bytes(const QrowParams& q, int blocks) {
 // registers costing a wave per SIMD.
 template <int P, int MT, int KW, bool F16>
 bool launch_w8a16_s_kw(const QrowParams& p, int blocks, hipStream_t s) {
-  const size_t xl = stream_xl_bytes(p, blocks);
+  const size_t xl = stream_xl_bytes(p, blocks, KW > 1 ? (size_t)KW * P * MT * 64 * sizeof(f32x4) : 0);
   if (xl) {
     hipLaunchKernelGGL((k_w8a16_s<P, MT, KW, 2, F16, true>), dim3(blocks), dim3(KW * 64), xl, s, p);
     return true;
@@ -1945,7 +1947,7 @@ int run_linears(QrowParams p, int x_dtype, int64_t M, hipStream_t s, bool row_st
       const bool f16 = x_dtype == QS_F16;
       // long rows with LDS-resident activations stream (few tiles, deep K); the rest
       // keep the round-based kernel, which measured faster for 1536-wide layers
-      if (q.K >= 4096 && stream_fits(q) && stream_xl_bytes(q, blocks)) {
+      if (q.K >= 4096 && stream_fits(q) && stream_xl_bytes(q, blocks, 0)) {
         const int kw = pick_kw_s(blocks, q.K, 1);
         bool done;
         if (mm <= 16)

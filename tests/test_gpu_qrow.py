@@ -212,6 +212,34 @@ def test_swiglu(dev, m, n, k):
     assert err <= BF16_TOL, err
 
 
+# Few weight tiles (so many K slices per workgroup) and 17 to 32 activation rows that nearly
+# fill the LDS: the staged rows and the slices' sums together must stay within a workgroup's
+# 160 KB (32 rows of 2048: 128.5 + 32 KB; 17 rows of 4096: 136.3 + 32 KB).  N % 4 != 0 keeps
+# the public functions on these kernels.
+@pytest.mark.parametrize("swiglu,m,n,k", [(True, 32, 1000, 2048), (True, 31, 1001, 2176), (True, 31, 200, 2048),
+                                          (False, 17, 1001, 4096), (False, 17, 301, 4224), (False, 16, 1001, 4480)])
+def test_streamed_rows_near_the_lds_limit(dev, swiglu, m, n, k):
+    q = _qrow()
+    rng, codes, scales = _case(n, k, seed=m + n)
+    _, codes2, scales2 = _case(n, k, seed=m + n + 1)
+    x = oq.round_bf16(rng.standard_normal((m, k)).astype(np.float32))
+    c, s, c2, s2 = (_dev(a, dev) for a in (codes, scales, codes2, scales2))
+    xd = _dev(x, dev, torch.bfloat16)
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+    if swiglu:
+        ref = oq.qrow_swiglu(codes, scales, codes2, scales2, x)
+        q.nat.call("qs_qrow_swiglu", xd.data_ptr(), k, c.data_ptr(), s.data_ptr(), c2.data_ptr(), s2.data_ptr(),
+                   y.data_ptr(), n, m, n, k, q.nat.stream_of(dev))
+        pub = q.fused_qrow_swiglu(q.CompactQRowPage("g", 0, n, k, c, s), q.CompactQRowPage("u", 0, n, k, c2, s2), xd)[0]
+    else:
+        ref = oq.qrow_matmul_w8a16(codes, scales, x)
+        q.nat.call("qs_qrow_matmul", xd.data_ptr(), q.nat.QS_BF16, k, c.data_ptr(), s.data_ptr(), y.data_ptr(), n, m, n,
+                   k, q.nat.stream_of(dev))
+        pub = q.qrow_matmul(c, s, xd)
+    assert oq.rel_l2(y.float().cpu().numpy(), ref) <= BF16_TOL
+    assert oq.rel_l2(pub.float().cpu().numpy(), ref) <= BF16_TOL
+
+
 @pytest.mark.parametrize("n,k", [(8960, 1536), (8193, 512), (12000, 256), (16384, 2048), (16385, 1040),
                                  (20000, 1536)])
 def test_swiglu_rows_equal_row_blocks(dev, n, k):
