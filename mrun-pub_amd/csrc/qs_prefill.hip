@@ -22,7 +22,7 @@ struct PfLin {
   int64_t ldy;
   int N;
   int tile_begin;  // first weight tile of this linear
-  int n_begin;     // first output column of this linear in the partial rows
+  int n_begin;     // first output column of this linear in the partial rows (a multiple of 4)
 };
 
 struct PfParams {
@@ -32,7 +32,7 @@ struct PfParams {
   int T, TS;  // 64-k steps, and steps per slice
   int S;      // slices
   int tiles_m, tiles_n;
-  int n_lin, n_total;
+  int n_lin, n_total;  // columns of a partial row: every linear's N rounded up to 4
   int vec;  // outputs allow 8-byte stores
   PfLin lin[4];
   float* part;  // [S][P][M][n_total] when S > 1
@@ -384,14 +384,9 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
       } else {
 #pragma unroll
         for (int pl = 0; pl < P; ++pl) {
-          float* pr = p.part + (((int64_t)s * P + pl) * p.M + m) * p.n_total + L0.n_begin + nb;
-          if (full) {
-            *reinterpret_cast<f32x4*>(pr) = sum[pl][j][t];
-          } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              if (nb + q < N) pr[q] = sum[pl][j][t][q];
-          }
+          // columns past N land in the row's padding
+          *reinterpret_cast<f32x4*>(p.part + (((int64_t)s * P + pl) * p.M + m) * p.n_total + L0.n_begin + nb) =
+              sum[pl][j][t];
         }
       }
     }
@@ -399,7 +394,9 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
 }
 
 // Slice sums in slice order and the epilogue: one thread per (row m, 4 columns of the
-// partial row); every linear's N is a multiple of 4 (the host checks).
+// partial row).  Partial rows hold every linear's columns rounded up to 4, so that any N can
+// be split (three fp32 rows of 1001 x 8960: 61 us in one slice, 15 in ten); the columns past N
+// are not stored.
 template <int P, int XT>
 __global__ __launch_bounds__(256) void k_prefill_reduce(PfParams p) {
   const int q4 = p.n_total / 4;
@@ -422,13 +419,16 @@ __global__ __launch_bounds__(256) void k_prefill_reduce(PfParams p) {
     for (int s = 1; s < p.S; ++s) a[pl] += *reinterpret_cast<const f32x4*>(pr + s * step);
   }
   const PfLin& L = p.lin[li];
+  const int n = ncol - L.n_begin;
+  const bool full = p.vec && n + 3 < L.N;
   if constexpr (XT == QS_F32) {
-    float* yr = static_cast<float*>(L.y) + (int64_t)m * L.ldy + (ncol - L.n_begin);
-    if (p.vec) {
+    float* yr = static_cast<float*>(L.y) + (int64_t)m * L.ldy + n;
+    if (full) {
       *reinterpret_cast<f32x4*>(yr) = a[0];
     } else {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) yr[q] = a[0][q];
+      for (int q = 0; q < 4; ++q)
+        if (n + q < L.N) yr[q] = a[0][q];
     }
     return;
   }
@@ -440,12 +440,13 @@ __global__ __launch_bounds__(256) void k_prefill_reduce(PfParams p) {
     for (int pl = 0; pl < P; ++pl) v[pl] = a[pl][q];
     o[q] = w8a16_out<P, XT == QS_F16>(v);
   }
-  uint16_t* yr = static_cast<uint16_t*>(L.y) + (int64_t)m * L.ldy + (ncol - L.n_begin);
-  if (p.vec) {
+  uint16_t* yr = static_cast<uint16_t*>(L.y) + (int64_t)m * L.ldy + n;
+  if (full) {
     *reinterpret_cast<uint2*>(yr) = make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
   } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) yr[q] = o[q];
+    for (int q = 0; q < 4; ++q)
+      if (n + q < L.N) yr[q] = o[q];
   }
 }
 
@@ -483,10 +484,7 @@ struct PfPlan {
 PfPlan pf_plan(bool f32, int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool split) {
   const int64_t T = K / 64;
   int64_t n_total = 0;
-  for (int i = 0; i < (P == 2 ? 1 : n_lin); ++i) {
-    n_total += N[i];
-    split = split && N[i] % 4 == 0;
-  }
+  for (int i = 0; i < (P == 2 ? 1 : n_lin); ++i) n_total += cdiv(N[i], 4) * 4;
   PfPlan best{0, 1, 0, n_total};
   float best_t = 0.f;
   for (int k = f32 ? kPfShapes16 : 0; k < (f32 ? kPfShapesAll : kPfShapes16); ++k) {
@@ -577,7 +575,7 @@ int run_prefill(const void* x, int x_dtype, int64_t ldx, int n_lin, const QrowPr
     p.lin[i] = PfLin{lin[i].codes, lin[i].scales, lin[i].y, lin[i].ldy, (int)N[i], (int)tb, (int)nb};
     if (P == 1) {
       tb += cdiv(N[i], 16 * sh.NTP * sh.WN);
-      nb += N[i];
+      nb += cdiv(N[i], 4) * 4;
     }
   }
   if (P == 2) pf_launch<2, QS_BF16>(p, plan.shape, s);

@@ -39,7 +39,7 @@ def _untouched(buf, m, n):
 
 
 # Tile edges (16/32/64/128 activation rows, 128 weight rows), ragged N (N % 4 != 0 also turns
-# the K split and the vector stores off), one to a few K steps, and K splits.
+# the vector stores off), one to a few K steps, and K splits.
 @pytest.mark.parametrize("m", [33, 64, 65, 129, 300])
 @pytest.mark.parametrize("n,k", [(5, 64), (127, 128), (129, 320), (256, 1536), (72, 8960), (1030, 1088)])
 @pytest.mark.parametrize("f16", [False, True])
@@ -173,3 +173,65 @@ def test_many_f32_rows_rule(dev):
     assert [m for m in range(1, 9) if not q._many_f32_rows(m, 8192)] == [1, 2]
     assert [m for m in range(1, 9) if not q._many_f32_rows(m, 12288)] == [1, 2]
     assert [m for m in range(1, 9) if not q._many_f32_rows(m, 16384)] == [1]
+
+
+def _exact(ws, x, dt, swiglu):
+    """The result rounded once from 64-bit sums of the weights a product uses (fp32: unrounded)."""
+    def mul(w):
+        return x.double() @ (w[0].float() * w[1][:, None]).to(dt).double().t()
+
+    if swiglu:
+        g, u = (mul(w).to(dt).double() for w in ws)
+        return ((g * torch.sigmoid(g)).to(dt).double() * u).to(dt).double()
+    return mul(ws[0]) if dt == torch.float32 else mul(ws[0]).to(dt).double()
+
+
+def _check_entry(dev, dt, m, ns, k, *, swiglu=False, split=True, ldx=None, pad=0, shift=0):
+    """``qs_qrow_*_prefill`` on rows of ``ldx`` elements (NaN past k) into rows of n + ``pad``
+    that start ``shift`` elements into their buffer."""
+    from mrun_pub_amd import qrow as q
+
+    nat = q.nat
+    g = torch.Generator(device=dev).manual_seed(m + sum(ns) + k)
+    ws = []
+    for n in ns * (2 if swiglu else 1):
+        c = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=dev, generator=g)
+        ws.append((c, (torch.rand(n, device=dev, generator=g) + 0.5) / (73 * k ** 0.5)))
+    ldx = ldx or k
+    xb = torch.full((m, ldx), float("nan"), dtype=dt, device=dev)
+    xb[:, :k] = torch.randn(m, k, device=dev, generator=g).to(dt)
+    bufs = [torch.full((shift + m * (n + pad),), 7.0, dtype=dt, device=dev) for n in ns]
+    ys = [b[shift:].view(m, n + pad) for b, n in zip(bufs, ns)]
+    n_arr, xdt, lib = nat.int64_array(ns), nat.dtype_code(dt), nat.load()
+    wsb = int(lib.qs_qrow_prefill_workspace_bytes(xdt, m, len(ns), n_arr, k, int(swiglu))) if split else 0
+    work = torch.full((wsb // 4 + 64,), float("nan"), device=dev) if wsb else None
+    if swiglu:
+        nat.call("qs_qrow_swiglu_prefill", xb.data_ptr(), ldx, *(t.data_ptr() for w in ws for t in w), ys[0].data_ptr(),
+                 ns[0] + pad, m, ns[0], k, nat.ptr(work), wsb, nat.stream_of(dev))
+    else:
+        nat.call("qs_qrow_matmul_prefill", xb.data_ptr(), xdt, ldx, len(ns), nat.pointer_array([c.data_ptr() for c, _ in ws]),
+                 nat.pointer_array([s.data_ptr() for _, s in ws]), nat.pointer_array([y.data_ptr() for y in ys]),
+                 nat.int64_array([n + pad for n in ns]), n_arr, m, k, nat.ptr(work), wsb, nat.stream_of(dev))
+    tol = 1e-6 if dt == torch.float32 else TOL
+    for i, (n, y, b) in enumerate(zip(ns, ys, bufs)):
+        ref = _exact(ws if swiglu else [ws[i]], xb[:, :k], dt, swiglu)
+        err = float((y[:, :n].double() - ref).norm() / ref.norm())
+        assert err <= tol, (n, err)
+        assert bool((b[:shift] == 7).all()) and bool((y[:, n:] == 7).all())
+    if work is not None:
+        assert bool(torch.isnan(work[wsb // 4:]).all())
+    return wsb
+
+
+# Ragged widths in K splits: partial rows hold each linear's columns rounded up to 4, alone, in
+# a SwiGLU and beside other linears; output rows that allow vector stores (N + pad a multiple of
+# 4, aligned) and rows that do not.
+@pytest.mark.parametrize("dt,m,ns,k,swiglu", [
+    (torch.float32, 3, [1001], 8960, False), (torch.float32, 37, [301, 6, 1], 1536, False),
+    (torch.bfloat16, 33, [1001], 8960, False), (torch.float16, 50, [3, 130, 65, 301], 4096, False),
+    (torch.bfloat16, 40, [301], 8192, True), (torch.bfloat16, 140, [66], 4096, True)])
+@pytest.mark.parametrize("vec", [False, True])
+def test_prefill_ragged_widths_split(dev, dt, m, ns, k, swiglu, vec):
+    pad = -ns[0] % 4 if vec and len(ns) == 1 else 0
+    assert _check_entry(dev, dt, m, ns, k, swiglu=swiglu, pad=pad) > 0
+    assert _check_entry(dev, dt, m, ns, k, swiglu=swiglu, pad=pad, split=False) == 0
