@@ -61,8 +61,8 @@ int qs_qrow_dequant_rows(const int8_t* codes, const float* scales, int64_t N, in
  *   x_dtype F32 : W in fp32, fp32 accumulate, y F32 (QStore fp32 compute contract).
  *   x_dtype BF16: W rounded to bf16 per element, fp32 accumulate, y BF16 (W8A16).
  *   x_dtype F16 : W rounded to fp16 per element, fp32 accumulate, y F16.
- * Few rows (decode) and fp32 use a VALU kernel, more rows an MFMA kernel; results agree
- * within the fp32-accumulation tolerance but are not bitwise batch invariant. */
+ * Few rows (decode) use a VALU kernel, more rows MFMA kernels; results agree within the
+ * fp32-accumulation tolerance but are not bitwise batch invariant. */
 int qs_qrow_matmul(const void* x, int x_dtype, int64_t ldx, const int8_t* codes,
                    const float* scales, void* y, int64_t ldy, int64_t M, int64_t N,
                    int64_t K, void* stream);
@@ -109,11 +109,18 @@ int qs_qrow_swiglu_batched(const void* x, int64_t ldx, const int8_t* gate_codes,
  * qs_qrow_swiglu in one launch over all M rows.  K % 64 == 0 and 16-byte aligned
  * activation and weight rows, otherwise QS_ERR_UNSUPPORTED.  The tile shape and the number
  * of K slices follow (M, N, K); the slices' fp32 partial sums are added in slice order.
- * qs_qrow_matmul, qs_qrow_matmul_multi and qs_qrow_swiglu take the same kernel, without a
- * K split, above 32 rows of BF16 / F16 and for batches of more than a few F32 rows.
+ * qs_qrow_matmul, qs_qrow_matmul_multi and qs_qrow_swiglu take the same kernel without a K
+ * split, for more than 32 rows of BF16 / F16 or a few of F32, where it is expected to be
+ * faster than theirs without one (mostly rows shorter than 4096, or more than 64 of them).
+ *   qs_qrow_prefill_plan (host only): the workspace bytes of a call that is expected to gain
+ *              from these entry points with a K split (split != 0) or without one, -1 where
+ *              the plain entry points' other kernels are; `tile` (nullable) receives the
+ *              activation rows and the weight rows of a tile, its K parts and the K slices.
  *   workspace: qs_qrow_prefill_workspace_bytes(x_dtype, M, n_linear, N, K, swiglu) bytes,
  *              16-byte aligned (0: K is not split; null also asks for no split), contents
  *              clobbered; calls that run concurrently need their own. */
+int64_t qs_qrow_prefill_plan(int x_dtype, int64_t M, int n_linear, const int64_t* N, int64_t K,
+                             int swiglu, int split, int32_t* tile);
 size_t qs_qrow_prefill_workspace_bytes(int x_dtype, int64_t M, int n_linear, const int64_t* N,
                                        int64_t K, int swiglu);
 int qs_qrow_matmul_prefill(const void* x, int x_dtype, int64_t ldx, int n_linear,

@@ -53,6 +53,7 @@ SIGNATURES: dict[str, tuple] = {
     "qs_qrow_batched_workspace_bytes": (ctypes.c_size_t, [_L, _I, _P, _L, _I]),
     "qs_qrow_matmul_batched": (_I, [_P, _I, _L, _I, _P, _P, _P, _P, _P, _L, _L, _P, ctypes.c_size_t, _P]),
     "qs_qrow_swiglu_batched": (_I, [_P, _L, _P, _P, _P, _P, _P, _L, _L, _L, _L, _P, ctypes.c_size_t, _P]),
+    "qs_qrow_prefill_plan": (_L, [_I, _L, _I, _P, _L, _I, _I, _P]),
     "qs_qrow_prefill_workspace_bytes": (ctypes.c_size_t, [_I, _L, _I, _P, _L, _I]),
     "qs_qrow_matmul_prefill": (_I, [_P, _I, _L, _I, _P, _P, _P, _P, _P, _L, _L, _P, ctypes.c_size_t, _P]),
     "qs_qrow_swiglu_prefill": (_I, [_P, _L, _P, _P, _P, _P, _P, _L, _L, _L, _L, _P, ctypes.c_size_t, _P]),

@@ -475,6 +475,7 @@ constexpr int64_t kPfMaxWorkspace = (int64_t)256 << 20;
 struct PfPlan {
   int shape, S;
   int64_t tiles_n, n_total;
+  float us;  // modelled time
 };
 
 // The shape and slice count with the smallest modelled time: a large tile reuses its operands
@@ -485,8 +486,7 @@ PfPlan pf_plan(bool f32, int64_t M, int n_lin, const int64_t* N, int64_t K, int 
   const int64_t T = K / 64;
   int64_t n_total = 0;
   for (int i = 0; i < (P == 2 ? 1 : n_lin); ++i) n_total += cdiv(N[i], 4) * 4;
-  PfPlan best{0, 1, 0, n_total};
-  float best_t = 0.f;
+  PfPlan best{0, 1, 0, n_total, 0.f};
   for (int k = f32 ? kPfShapes16 : 0; k < (f32 ? kPfShapesAll : kPfShapes16); ++k) {
     const PfShape& sh = kPfShapes[k];
     int64_t tiles_n = 0;
@@ -500,10 +500,7 @@ PfPlan pf_plan(bool f32, int64_t M, int n_lin, const int64_t* N, int64_t K, int 
       const float rounds = (float)cdiv(cdiv(T, S), sh.WK);
       float t = kPfLaunch + rounds * std::max(sh.lat, sh.thr * per_cu) + sh.end * per_cu;
       if (S > 1) t += kPfReduce + 2.f * (float)part / kPfReduceBytes;
-      if (best.tiles_n == 0 || t < best_t) {
-        best = PfPlan{k, S, tiles_n, n_total};
-        best_t = t;
-      }
+      if (best.tiles_n == 0 || t < best.us) best = PfPlan{k, S, tiles_n, n_total, t};
     }
   }
   return best;
@@ -530,6 +527,44 @@ void pf_launch(const PfParams& p, int shape, hipStream_t s) {
 }
 
 }  // namespace
+
+// Whether the prefill kernel is expected to beat the launches that qs_qrow_matmul_multi and
+// qs_qrow_swiglu otherwise make, from `split` or unsplit plan times against their times in
+// microseconds (graph replays, 2 to 512 rows of the shapes below and their K and N in other
+// pairs).  K that those kernels do not take runs one wave per weight row there: always prefill.
+bool prefill_faster(int x_dtype, int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool split) {
+  if (M < 2) return false;
+  float rows = 0.f;  // millions of weights
+  for (int i = 0; i < (P == 2 ? 1 : n_lin); ++i) rows += (float)N[i];
+  const float k = (float)K * 1e-3f, nk = rows * k * 1e-3f;
+  if (x_dtype == QS_F32) {
+    // One launch of the VALU kernel per 4, 2 or 1 rows that fit its 64 KiB (none past 12288):
+    // 13% rms over 91 products.  It keeps rows of a single launch, two rows and, beside a split, those
+    // the plan does not win by 4 us: a split call asks for a workspace and launches twice, 6 us
+    // more of host time than the plain call (eager calls of 8 rows of 4096 x 1024 12.6 against
+    // 18.4 us for 10.2 and 9.1 on the GPU; 6 rows of 4096 x 4096 21.6 against 18.7; 3 rows of
+    // 1536 x 8960 16.2 against 18.9, and 61 on the GPU unsplit).
+    if (K > 12288) return true;
+    const int mb = valu_mb(x_dtype, K, M);
+    const float L = (float)cdiv(M, mb);
+    if (L < 2.f || M < 3) return false;
+    const float valu = 0.65f + L * (2.6f + nk * (0.115f * mb - 0.019f) + 0.149f * mb * k);
+    return pf_plan(true, M, n_lin, N, K, P, split).us + (split ? 4.f : 0.f) < valu;
+  }
+  // 16-bit: 32-row batches.  Past two of them, with a split, for a SwiGLU (33 rows of
+  // 8960 x 1536 28 -> 14.5 us; at worst 37 -> 39, 33 rows of 301 x 8192 unsplit) and for rows
+  // they do not take the prefill kernel is faster; unsplit it is bound by its K steps up to 64
+  // rows (33 rows of 1536 x 8960 42 us against 33, of 4096 x 4096 22 against 20, of
+  // 14336 x 4096 29 against 62), where a batch takes 2.7 us and its K steps or its weights.
+  // Weights past the L2s' 32 MB slow the steps of the plan by a fifth (48 rows of
+  // 4096 x 14336 82 us against 68).
+  if (M <= 32) return false;
+  if (M > 64 || split || P == 2 || K % 128 != 0) return true;
+  const float body = std::max(2.4f * k, 0.7f * nk);
+  const int tail = (int)M - 32;
+  const float batches = 5.4f + body * (tail > 16 ? 2.f : 1.33f + 0.022f * (float)tail);
+  return pf_plan(false, M, n_lin, N, K, P, false).us * (nk > 32.f ? 1.2f : 1.f) < batches;
+}
 
 // y = x @ W^T over the linears' shared x: `lin` holds the P planes of a SwiGLU (P = 2, y in lin[0])
 // or n_lin linears.  `workspace` null: no K split.  Returns QS_ERR_UNSUPPORTED, without a
@@ -588,6 +623,22 @@ int run_prefill(const void* x, int x_dtype, int64_t ldx, int n_lin, const QrowPr
 }  // namespace qs
 
 using namespace qs;
+
+extern "C" int64_t qs_qrow_prefill_plan(int x_dtype, int64_t M, int n_linear, const int64_t* N, int64_t K, int swiglu,
+                                        int split, int32_t* tile) {
+  if (!N || n_linear < 1 || n_linear > 4 || M < 1 || K < 64) return -1;
+  const int P = swiglu ? 2 : 1;
+  const PfPlan plan = pf_plan(x_dtype == QS_F32, M, n_linear, N, K, P, split != 0);
+  if (tile) {
+    const PfShape& sh = kPfShapes[plan.shape];
+    tile[0] = 16 * sh.MT;
+    tile[1] = 16 * sh.NTP / P * sh.WN;
+    tile[2] = sh.WK;
+    tile[3] = plan.S;
+  }
+  if (!prefill_faster(x_dtype, M, n_linear, N, K, P, split != 0)) return -1;
+  return plan.S > 1 ? plan.S * P * M * plan.n_total * 4 : 0;
+}
 
 extern "C" size_t qs_qrow_prefill_workspace_bytes(int x_dtype, int64_t M, int n_linear, const int64_t* N, int64_t K,
                                                   int swiglu) {

@@ -1733,17 +1733,6 @@ int validate_common(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t 
   return QS_OK;
 }
 
-constexpr int kLdsBudget = 64 * 1024;
-
-// Activation rows per VALU launch: the largest of 4/2/1 whose LDS copy fits.
-int valu_mb(int x_dtype, int64_t K, int64_t M) {
-  const int es = x_dtype == QS_F32 ? 4 : 2;
-  const int cap = x_dtype == QS_F32 ? 4 : 2;
-  for (int mb = cap; mb >= 1; mb /= 2)
-    if ((int64_t)mb * K * es <= kLdsBudget && (mb <= M || mb == 1)) return mb;
-  return 0;
-}
-
 bool valu_eligible(const QrowParams& p, int x_dtype) {
   const int es = x_dtype == QS_F32 ? 4 : 2;
   if (p.K % 16 != 0 || (p.ldx * es) % 16 != 0 || !aligned(p.x, 16)) return false;
@@ -1904,16 +1893,14 @@ void launch_top2_mb(const QrowParams& q, int rows, int start_row, float* pv, int
 // blocks; the fused path uses 8-row blocks, so this bounds both).
 int64_t top2_blocks(int64_t rows) { return cdiv(rows, 4); }
 
-// Whether a call takes the prefill kernel: 16-bit rows past a 32-row batch; fp32 rows that
-// would need three VALU launches, or two for three or more rows (4096 x 1024: three rows
-// 8.4 -> 8.1 us, two 7.1 against 8.1; 1536 x 8960: three rows 17.8 -> 15.5, two 11.7 against
-// 15.6).  Single rows always keep the decode kernels.
+// Whether a call takes the prefill kernel, which has no workspace here and so no K split: rows
+// that neither of this file's fast kernels takes, or that it is expected to run faster.
 bool many_rows(const QrowParams& p, int x_dtype, int64_t M) {
-  if (x_dtype != QS_F32) return M > 32;
-  if (M < 2) return false;
-  if (!valu_eligible(p, x_dtype)) return true;
-  const int64_t launches = cdiv(M, valu_mb(x_dtype, p.K, M));
-  return launches >= 3 || (launches == 2 && M >= 3);
+  if (M < 2 || (x_dtype != QS_F32 && M <= 32)) return false;
+  if (x_dtype == QS_F32 && !valu_eligible(p, x_dtype)) return true;
+  int64_t N[4];
+  for (int i = 0; i < p.n_lin; ++i) N[i] = p.lin[i].N;
+  return prefill_faster(x_dtype, M, p.n_lin, N, p.K, 1, false);
 }
 
 // Runs one set of linears sharing x.

@@ -1,4 +1,4 @@
-// Pieces shared by the MFMA qrow kernels (qs_batched.hip, qs_prefill.hip).
+// Pieces shared by the qrow kernels (qs_qrow.hip, qs_batched.hip, qs_prefill.hip).
 #pragma once
 
 #include "qs_common.h"
@@ -41,6 +41,17 @@ __device__ __forceinline__ uint16_t w8a16_out(const float (&v)[P]) {
   }
 }
 
+constexpr int kLdsBudget = 64 * 1024;  // activation rows staged by the VALU kernels
+
+// Activation rows per VALU launch: the largest of 4/2/1 whose LDS copy fits.
+inline int valu_mb(int x_dtype, int64_t K, int64_t M) {
+  const int es = x_dtype == QS_F32 ? 4 : 2;
+  const int cap = x_dtype == QS_F32 ? 4 : 2;
+  for (int mb = cap; mb >= 1; mb /= 2)
+    if ((int64_t)mb * K * es <= kLdsBudget && (mb <= M || mb == 1)) return mb;
+  return 0;
+}
+
 // One linear of a call with many activation rows (qs_prefill.hip).
 struct QrowPrefillLin {
   const int8_t* codes;
@@ -49,6 +60,7 @@ struct QrowPrefillLin {
   int64_t ldy;
   int64_t N;
 };
+bool prefill_faster(int x_dtype, int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool split);
 int run_prefill(const void* x, int x_dtype, int64_t ldx, int n_lin, const QrowPrefillLin* lin, int P, int64_t M,
                 int64_t K, void* workspace, size_t workspace_bytes, hipStream_t s);
 

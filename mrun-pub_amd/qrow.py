@@ -183,9 +183,10 @@ def _batched_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool 
 
 
 def _many_f32_rows(m: int, k: int) -> bool:
-    """fp32 rows that take the prefill kernel: those that would need three launches of the VALU
-    kernel (which stages 4, 2 or 1 rows of k floats in 64 KiB of LDS; none past k = 12288), or
-    two for three or more rows.  The C entry points' rule, with its timings, is many_rows()."""
+    """fp32 rows that may gain from the prefill kernel: those that would need three launches of
+    the VALU kernel (which stages 4, 2 or 1 rows of k floats in 64 KiB of LDS; none past
+    k = 12288), or two for three or more rows.  Whether they do depends on the widths too:
+    ``qs_qrow_prefill_plan`` decides."""
     if m < 2 or k > 12288:
         return m >= 2
     mb = next((b for b in (4, 2) if b * k * 4 <= 65536 and b <= m), 1)
@@ -194,8 +195,9 @@ def _many_f32_rows(m: int, k: int) -> bool:
 
 
 def _prefill_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool = False) -> bool:
-    """More rows than the decode and batched kernels take, in the layout qs_qrow_matmul_prefill
-    does (rows of whole 64-k steps, 16-byte aligned; offsets inside a 128-row tile are 31-bit)."""
+    """Whether qs_qrow_matmul_prefill takes a call of more rows than the decode and batched
+    kernels do: rows of whole 64-k steps, 16-byte aligned; offsets inside a 128-row tile are
+    31-bit."""
     m, k = int(x2.shape[0]), int(x2.shape[1])
     many = _many_f32_rows(m, k) if x2.dtype == torch.float32 else m > BATCHED_MAX_M
     return (many and (not swiglu or x2.dtype == torch.bfloat16) and k % 64 == 0 and k < 1 << 22
@@ -205,38 +207,40 @@ def _prefill_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool 
 def _run_batched(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
                  swiglu: bool) -> None:
     """At most 32 16-bit rows through the batched kernels (the split depends on N and K only)."""
-    _run_many("batched", x2, pages, outs, swiglu)
+    ns = nat.int64_array([int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]])
+    _run_many("batched", x2, pages, outs, swiglu, ns,
+              int(nat.load().qs_qrow_batched_workspace_bytes(x2.shape[0], len(ns), ns, x2.shape[1], int(swiglu))))
 
 
 def _run_prefill(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
-                 swiglu: bool) -> None:
-    """Any number of rows through the prefill kernel."""
-    _run_many("prefill", x2, pages, outs, swiglu)
+                 swiglu: bool) -> bool:
+    """Any number of rows through the prefill kernel; ``False``, with nothing launched, where
+    the kernels of the plain entry points are expected to be faster."""
+    ns = nat.int64_array([int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]])
+    ws_bytes = int(nat.load().qs_qrow_prefill_plan(nat.dtype_code(x2.dtype), x2.shape[0], len(ns), ns, x2.shape[1],
+                                                   int(swiglu), 1, None))
+    if ws_bytes < 0:
+        return False
+    _run_many("prefill", x2, pages, outs, swiglu, ns, ws_bytes)
+    return True
 
 
 def _run_many(kind: str, x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
-              swiglu: bool) -> None:
+              swiglu: bool, ns, ws_bytes: int) -> None:
     """``qs_qrow_matmul_<kind>`` / ``qs_qrow_swiglu_<kind>`` with a workspace for the K-slice
     partial sums."""
     device = x2.device
     m, k = int(x2.shape[0]), int(x2.shape[1])
-    ns = [int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]]
     stream = nat.stream_of(device)
-    n_arr = nat.int64_array(ns)
-    lib, xdt = nat.load(), nat.dtype_code(x2.dtype)
-    if kind == "batched":
-        ws_bytes = int(lib.qs_qrow_batched_workspace_bytes(m, len(ns), n_arr, k, int(swiglu)))
-    else:
-        ws_bytes = int(lib.qs_qrow_prefill_workspace_bytes(xdt, m, len(ns), n_arr, k, int(swiglu)))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
     if swiglu:
         (gc, gs), (uc, us) = pages
         nat.call(f"qs_qrow_swiglu_{kind}", nat.ptr(x2), k, nat.ptr(gc), nat.ptr(gs), nat.ptr(uc), nat.ptr(us),
                  nat.ptr(outs[0]), ns[0], m, ns[0], k, nat.ptr(ws), ws_bytes, stream)
     else:
-        nat.call(f"qs_qrow_matmul_{kind}", nat.ptr(x2), xdt, k, len(pages),
+        nat.call(f"qs_qrow_matmul_{kind}", nat.ptr(x2), nat.dtype_code(x2.dtype), k, len(pages),
                  nat.pointer_array([nat.ptr(c) for c, _ in pages]), nat.pointer_array([nat.ptr(sc) for _, sc in pages]),
-                 nat.pointer_array([nat.ptr(o) for o in outs]), n_arr, n_arr, m, k, nat.ptr(ws), ws_bytes, stream)
+                 nat.pointer_array([nat.ptr(o) for o in outs]), ns, ns, m, k, nat.ptr(ws), ws_bytes, stream)
 
 
 @nat.inference
@@ -264,8 +268,9 @@ def qrow_matmul(
     y = _out_buffer(out, m, n, x.dtype, device)
     if m > 1 and not row_stable and _batched_eligible(flat, [codes]):
         _run_batched(flat, [(codes, scales)], [y], swiglu=False)
-    elif m > 1 and not row_stable and _prefill_eligible(flat, [codes]):
-        _run_prefill(flat, [(codes, scales)], [y], swiglu=False)
+    elif (m > 1 and not row_stable and _prefill_eligible(flat, [codes])
+          and _run_prefill(flat, [(codes, scales)], [y], swiglu=False)):
+        pass
     elif m:
         nat.call(
             "qs_qrow_matmul_row_stable" if row_stable else "qs_qrow_matmul",
@@ -307,8 +312,9 @@ def qrow_matmul_multi(
     outs = [_out_buffer(None if out is None else out[i], m, n, x.dtype, device) for i, (n, _) in enumerate(shapes)]
     if m > 1 and _batched_eligible(flat, [c for c, _ in pages]):
         _run_batched(flat, pages, outs, swiglu=False)
-    elif m > 1 and _prefill_eligible(flat, [c for c, _ in pages]):
-        _run_prefill(flat, pages, outs, swiglu=False)
+    elif (m > 1 and _prefill_eligible(flat, [c for c, _ in pages])
+          and _run_prefill(flat, pages, outs, swiglu=False)):
+        pass
     elif m:
         nat.call(
             "qs_qrow_matmul_multi",
@@ -406,8 +412,10 @@ def qrow_swiglu_into(gate_page: CompactQRowPage, up_page: CompactQRowPage, activ
     y = _out_buffer(out, m, n, torch.bfloat16, device)
     if m > 1 and _batched_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
         _run_batched(flat, [(gate_page.codes, gate_page.scales), (up_page.codes, up_page.scales)], [y], swiglu=True)
-    elif m > 1 and _prefill_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True):
-        _run_prefill(flat, [(gate_page.codes, gate_page.scales), (up_page.codes, up_page.scales)], [y], swiglu=True)
+    elif (m > 1 and _prefill_eligible(flat, [gate_page.codes, up_page.codes], swiglu=True)
+          and _run_prefill(flat, [(gate_page.codes, gate_page.scales), (up_page.codes, up_page.scales)], [y],
+                           swiglu=True)):
+        pass
     elif m:
         nat.call(
             "qs_qrow_swiglu",

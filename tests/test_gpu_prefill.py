@@ -166,9 +166,18 @@ def test_prefill_fp32_long_rows_and_range(dev):
 
 
 def test_many_f32_rows_rule(dev):
-    """Which fp32 row counts leave the decode kernel: the Python rule equals the C one."""
+    """Which fp32 row counts leave the decode kernel: the binding's early answer never differs
+    from the library's (whose rule looks at the widths too)."""
     from mrun_pub_amd import qrow as q
 
+    for k in (64, 1024, 4096, 4160, 8192, 8256, 12288, 12352, 16384):
+        for m in range(1, 12):
+            plans = [q.nat.load().qs_qrow_prefill_plan(q.nat.QS_F32, m, 1, q.nat.int64_array([n]), k, 0, 1, None)
+                     for n in (1, 300, 4096, 60000)]
+            if not q._many_f32_rows(m, k):
+                assert plans == [-1] * 4, (m, k)
+            elif k > 12288:
+                assert min(plans) >= 0, (m, k)
     assert [m for m in range(1, 9) if not q._many_f32_rows(m, 1024)] == [1, 2, 4]
     assert [m for m in range(1, 9) if not q._many_f32_rows(m, 8192)] == [1, 2]
     assert [m for m in range(1, 9) if not q._many_f32_rows(m, 12288)] == [1, 2]

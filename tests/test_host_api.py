@@ -85,3 +85,33 @@ def test_row_id_normalisation():
         normalize_row_ids([-5], 4)
     with pytest.raises(TypeError):
         normalize_row_ids([0.5], 4)
+
+
+def test_prefill_plan_follows_widths_and_split():
+    """The many-row kernel is left alone where the decode kernels are faster: long rows of few
+    columns without a K split, and few fp32 rows."""
+    import mrun_pub_amd._native as nat
+
+    if not nat.LIB_PATH.exists():
+        pytest.skip("library not built")
+
+    def plan(dt, m, ns, k, split, swiglu=0):
+        return nat.load().qs_qrow_prefill_plan(dt, m, len(ns), nat.int64_array(ns), k, swiglu, split, None)
+
+    f32, bf16 = nat.QS_F32, nat.QS_BF16
+    # without a split (measured, decode kernels against this one): 16 / 61 us, 26 / 62, 33 / 42, 57 / 81, 68 / 82,
+    # 20 / 22
+    for dt, m, n, k in ((f32, 3, 1536, 8960), (f32, 5, 1001, 8960), (bf16, 33, 1536, 8960), (bf16, 33, 4096, 14336),
+                        (bf16, 48, 4096, 14336), (bf16, 33, 4096, 4096)):
+        assert plan(dt, m, [n], k, 0) == -1, (m, n, k)
+    # 81 / 61, 19 / 10, 62 / 29, 77 / 43, 22 / 12
+    for dt, m, n, k in ((f32, 16, 1536, 8960), (f32, 16, 4096, 1024), (bf16, 33, 14336, 4096), (bf16, 96, 1536, 8960),
+                        (bf16, 33, 8960, 1536)):
+        assert plan(dt, m, [n], k, 0) == 0, (m, n, k)
+    # with one: 26 / 16, 20 / 15, 33 / 15; eager calls of few short fp32 rows 12 / 18
+    assert plan(f32, 5, [1536], 8960, 1) > 0 and plan(f32, 5, [4096], 4096, 1) > 0
+    assert plan(bf16, 33, [1001], 8960, 1) > 0
+    assert plan(f32, 3, [4096], 1024, 1) == -1 and plan(f32, 8, [4096], 1024, 1) == -1
+    # several linears count together
+    assert plan(f32, 3, [14336, 14336], 4096, 0) == 0 and plan(f32, 3, [256, 256], 4096, 0) == -1
+    assert plan(bf16, 33, [1536], 8960, 0, swiglu=1) == 0
