@@ -526,6 +526,13 @@ void pf_launch(const PfParams& p, int shape, hipStream_t s) {
   }
 }
 
+// Activation rows that one launch of a plan takes: a grid has fewer than 2^32 threads (32-row
+// fp32 tiles of one column reach that at 2^28 rows).  0: not even one tile row.
+int64_t pf_launch_rows(const PfPlan& plan) {
+  const PfShape& sh = kPfShapes[plan.shape];
+  return (int64_t)UINT32_MAX / (sh.WN * sh.WK * 64) / (plan.tiles_n * plan.S) * 16 * sh.MT;
+}
+
 }  // namespace
 
 // Whether the prefill kernel is expected to beat the launches that qs_qrow_matmul_multi and
@@ -590,16 +597,13 @@ int run_prefill(const void* x, int x_dtype, int64_t ldx, int n_lin, const QrowPr
       return fail(QS_ERR_INVALID, "qrow prefill: workspace smaller than qs_qrow_prefill_workspace_bytes()");
     if (!aligned(workspace, 16)) return fail(QS_ERR_INVALID, "qrow prefill: workspace must be 16-byte aligned");
   }
-  const int64_t tiles_m = cdiv(M, 16 * sh.MT);
-  if (tiles_m * plan.tiles_n * plan.S > INT_MAX || plan.n_total > INT_MAX) return QS_ERR_UNSUPPORTED;
-  p.x = x;
+  const int64_t rows = pf_launch_rows(plan);
+  if (rows == 0 || plan.n_total > INT_MAX) return QS_ERR_UNSUPPORTED;
   p.ldx = ldx;
-  p.M = (int)M;
   p.K = (int)K;
   p.T = (int)(K / 64);
   p.S = plan.S;
   p.TS = (int)cdiv(p.T, plan.S);
-  p.tiles_m = (int)tiles_m;
   p.tiles_n = (int)plan.tiles_n;
   p.n_lin = n_lin;
   p.n_total = (int)plan.n_total;
@@ -613,10 +617,17 @@ int run_prefill(const void* x, int x_dtype, int64_t ldx, int n_lin, const QrowPr
       nb += cdiv(N[i], 4) * 4;
     }
   }
-  if (P == 2) pf_launch<2, QS_BF16>(p, plan.shape, s);
-  else if (f32) pf_launch<1, QS_F32>(p, plan.shape, s);
-  else if (x_dtype == QS_F16) pf_launch<1, QS_F16>(p, plan.shape, s);
-  else pf_launch<1, QS_BF16>(p, plan.shape, s);
+  for (int64_t m0 = 0; m0 < M; m0 += rows) {
+    p.M = (int)std::min(rows, M - m0);
+    p.tiles_m = (int)cdiv(p.M, 16 * sh.MT);
+    p.x = static_cast<const char*>(x) + m0 * ldx * es;
+    for (int i = 0; i < n_lin; ++i)
+      if (lin[i].y) p.lin[i].y = static_cast<char*>(lin[i].y) + m0 * lin[i].ldy * es;
+    if (P == 2) pf_launch<2, QS_BF16>(p, plan.shape, s);
+    else if (f32) pf_launch<1, QS_F32>(p, plan.shape, s);
+    else if (x_dtype == QS_F16) pf_launch<1, QS_F16>(p, plan.shape, s);
+    else pf_launch<1, QS_BF16>(p, plan.shape, s);
+  }
   return hip_check(hipGetLastError(), "k_prefill launch");
 }
 
@@ -636,6 +647,7 @@ extern "C" int64_t qs_qrow_prefill_plan(int x_dtype, int64_t M, int n_linear, co
     tile[2] = sh.WK;
     tile[3] = plan.S;
   }
+  if (pf_launch_rows(plan) == 0 || plan.n_total > INT_MAX) return -1;
   if (!prefill_faster(x_dtype, M, n_linear, N, K, P, split != 0)) return -1;
   return plan.S > 1 ? plan.S * P * M * plan.n_total * 4 : 0;
 }

@@ -244,3 +244,28 @@ def test_prefill_ragged_widths_split(dev, dt, m, ns, k, swiglu, vec):
     pad = -ns[0] % 4 if vec and len(ns) == 1 else 0
     assert _check_entry(dev, dt, m, ns, k, swiglu=swiglu, pad=pad) > 0
     assert _check_entry(dev, dt, m, ns, k, swiglu=swiglu, pad=pad, split=False) == 0
+
+
+def test_prefill_rows_past_one_launch(dev):
+    """More rows than one grid's 2^32 threads hold: 32-row tiles of one column reach that at 2^28
+    rows (a 69 GB input).  All rows are zero but a few on both sides of every edge."""
+    from mrun_pub_amd import qrow as q
+
+    m, k = 2**28 + 40, 64
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("needs 80 GB of free device memory")
+    codes, scales = _case(1, k, seed=1)
+    c, s = torch.from_numpy(codes).to(dev), torch.from_numpy(scales).to(dev)
+    tile = (q.nat.ctypes.c_int32 * 4)()
+    assert q.nat.load().qs_qrow_prefill_plan(q.nat.QS_F32, m, 1, q.nat.int64_array([1]), k, 0, 1, tile) == 0
+    assert m // tile[0] * 512 >= 2**32  # (8 waves per workgroup)
+    rows = torch.tensor([0, 31, 32, 2**28 - 65, 2**28 - 33, 2**28 - 32, 2**28 - 1, 2**28, m - 1], device=dev)
+    some = torch.randn(len(rows), k, device=dev, generator=torch.Generator(device=dev).manual_seed(2))
+    x = torch.zeros(m, k, device=dev)
+    x[rows] = some
+    y = q.qrow_matmul(c, s, x)
+    del x
+    ref = some.double() @ (c.double() * s.double()[:, None]).t()
+    assert float((y[rows].double() - ref).norm() / ref.norm()) <= 1e-6
+    assert int(torch.count_nonzero(y)) == len(rows)
+    torch.cuda.empty_cache()
