@@ -370,7 +370,9 @@ int qs_lowbit_dequant(const uint8_t* packed, int64_t row_bytes, const void* scal
                       int scale_dtype, const void* zeros, int zero_dtype, float offset, int bits,
                       int group_size, float* out, int64_t N, int64_t K, void* stream);
 
-/* Workspace bytes qs_lowbit_gemv needs for these dimensions. */
+/* Workspace bytes qs_lowbit_gemv needs for these dimensions: about 512 N + 32 K for a few rows;
+ * more rows share a launch with up to 128 MB of partial sums (BF16) or 256 + 64 MB of sums and
+ * split activations (F32), and with the bytes of a single row they still run, in more launches. */
 size_t qs_lowbit_workspace_bytes(int x_dtype, int64_t M, int64_t N, int64_t K, int group_size);
 
 /* Replaces QStoreInt3.matmul / QStoreInt2.matmul (qstore.py:1318-1341, 1451-1474):

@@ -374,14 +374,23 @@ void lg_launch(const LgParams& p, int mt, hipStream_t s) {
   else hipLaunchKernelGGL((k_lowbit_gemm<BITS, G, SZ, 4, 1>), grid, dim3(256), 0, s, p);
 }
 
-constexpr int64_t kLgTermRows = 512;  // fp32 activation rows per launch (three bf16 rows each)
+// Activation rows per launch.  fp32 (three bf16 rows each): at most 512, and no more than keep
+// the terms' partial sums within 256 MB and the terms within 64 MB (147 rows of a
+// 151,936 x 1536 head, where 512 would take 0.9 GB), but 32 in any case (384 bytes per weight
+// row, less than the 512 of a single row's workspace).  bf16: a grid has fewer than 2^32
+// threads (a K split's partial sums, at most kLgMaxPart, keep it far below).
+int64_t lg_chunk_rows(bool f32, int64_t N, int64_t K) {
+  if (!f32) return (int64_t)UINT32_MAX / 256 / cdiv(N, 64) * 32;
+  const int64_t rows = std::min(((int64_t)256 << 20) / (12 * N), ((int64_t)64 << 20) / (6 * K));
+  return std::min<int64_t>(512, std::max<int64_t>(32, rows));
+}
 
 }  // namespace
 
 size_t lowbit_gemm_workspace(int x_dtype, int64_t M, int64_t N, int64_t K, int G) {
   if (G != 64 && G != 128) return 0;
   if (x_dtype == QS_F32) {
-    const int64_t rows = 3 * std::min(M, kLgTermRows);
+    const int64_t rows = 3 * std::min(M, lg_chunk_rows(true, N, K));
     const LgPlan plan = lg_plan(rows, N, K, G, kLgMaxPart);
     return (size_t)((rows * K * 2 + 255) / 256 * 256) + (size_t)plan.S * rows * N * 4;
   }
@@ -415,8 +424,9 @@ int run_lowbit_gemm(const LowbitGemm& a, void* workspace, size_t workspace_bytes
   p.pair_mask = pc.pair_mask;
   p.pair_base = pc.pair_base;
   const int rpx = f32 ? 3 : 1;
-  const int64_t chunk = f32 ? kLgTermRows : a.M;
-  const int64_t xb_bytes = f32 ? (3 * std::min(a.M, chunk) * a.K * 2 + 255) / 256 * 256 : 0;
+  const int64_t chunk = std::min(a.M, lg_chunk_rows(f32, a.N, a.K));
+  if (chunk == 0 || chunk * rpx > INT_MAX) return QS_ERR_UNSUPPORTED;
+  const int64_t xb_bytes = f32 ? (3 * chunk * a.K * 2 + 255) / 256 * 256 : 0;
   if ((int64_t)workspace_bytes < xb_bytes) return QS_ERR_UNSUPPORTED;
   const int64_t room = (int64_t)workspace_bytes - xb_bytes;
   float* part = reinterpret_cast<float*>(static_cast<char*>(workspace) + xb_bytes);
@@ -424,7 +434,6 @@ int run_lowbit_gemm(const LowbitGemm& a, void* workspace, size_t workspace_bytes
     const int64_t mm = std::min(chunk, a.M - m0), rows = rpx * mm;
     if (f32 && room < rows * a.N * 4) return m0 ? fail(QS_ERR_INVALID, "lowbit_gemv: workspace too small") : QS_ERR_UNSUPPORTED;
     const LgPlan plan = lg_plan(rows, a.N, a.K, a.G, std::min(room, kLgMaxPart));
-    if (cdiv(rows, 16 * plan.MT) * p.tiles_n * plan.S > INT_MAX || rows > INT_MAX) return QS_ERR_UNSUPPORTED;
     p.M = (int)rows;
     p.S = plan.S;
     p.TS = (int)cdiv(p.T, plan.S);

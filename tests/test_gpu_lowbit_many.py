@@ -95,3 +95,15 @@ def test_many_rows_nonfinite_stays_in_its_row(dev):
     rows = np.array([r for r in range(40) if r not in (3, 39)])
     assert np.isfinite(y[rows]).all() and not np.isfinite(y[3]).any() and np.isnan(y[39]).all()
     assert oq.rel_l2(y[rows], ref(x[rows])) <= TOL
+
+
+def test_many_fp32_rows_of_a_wide_block(dev):
+    """A block so wide that its partial sums, not the 512 rows, end a launch (319 rows here)."""
+    from mrun_pub_amd.lowbit import lowbit_matmul
+
+    page, ref = _page(2, 64, True, 70001, 128, dev, seed=9)
+    x = np.random.default_rng(3).standard_normal((330, 128)).astype(np.float32)
+    y = lowbit_matmul(page, torch.from_numpy(x).to(dev)).cpu().numpy()
+    want = ref(x)
+    for rows in (slice(0, 319), slice(319, 330)):
+        assert oq.rel_l2(y[rows], want[rows]) <= TOL

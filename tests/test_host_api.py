@@ -115,3 +115,18 @@ def test_prefill_plan_follows_widths_and_split():
     # several linears count together
     assert plan(f32, 3, [14336, 14336], 4096, 0) == 0 and plan(f32, 3, [256, 256], 4096, 0) == -1
     assert plan(bf16, 33, [1536], 8960, 0, swiglu=1) == 0
+
+
+@pytest.mark.parametrize("dtype", ["QS_F32", "QS_BF16"])
+@pytest.mark.parametrize("n,k", [(151936, 1536), (11008, 4096), (4096, 11008), (1 << 22, 128), (512, 1 << 20)])
+def test_lowbit_workspace_is_bounded(dtype, n, k):
+    """Many rows of a wide block share a launch only as far as a bounded workspace allows."""
+    import mrun_pub_amd._native as nat
+
+    if not nat.LIB_PATH.exists():
+        pytest.skip("library not built")
+    size = nat.load().qs_lowbit_workspace_bytes
+    one = size(getattr(nat, dtype), 1, n, k, 64)
+    for m in (17, 149, 512, 4096, 100000):
+        # partial sums and split rows, or what a single row takes
+        assert size(getattr(nat, dtype), m, n, k, 64) <= max((256 + 64) << 20, one + 192 * k) + 512, m
