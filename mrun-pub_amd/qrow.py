@@ -473,6 +473,9 @@ def fused_qrow_top2(
     semantic prefix of the page per activation row (int32 global row indices, fp32
     logits), without materializing logits.  ``require_triton`` and the tile arguments
     keep the reference's signature and checks; the native kernel picks its own tiles.
+
+    Calls of one or two 16-bit rows (up to four fp32) and calls of more rows sum a logit in
+    different orders, so near ties may be ordered differently in a larger batch.
     """
     del require_triton
     _check_head(page, activations)
@@ -558,7 +561,9 @@ def fused_qrow_reranked_argmax(
     block_n: int = 64,
 ) -> tuple[torch.Tensor, torch.Tensor, str, int]:
     """Drop-in for ``fused_qrow_reranked_argmax`` (dense_qstore_cuda.py:1332-1374): fused
-    top-two search, then fp32 reranking of the two candidates."""
+    top-two search, then fp32 reranking of the two candidates (the same for a candidate
+    whatever the batch; which two it gets can depend on it in a near tie, see
+    :func:`fused_qrow_top2`)."""
     candidates, _, implementation, working = fused_qrow_top2(
         page, activations, semantic_row_count=semantic_row_count, require_triton=require_triton,
         block_m=block_m, block_n=block_n,

@@ -57,3 +57,28 @@ def test_head_top2_nonfinite_rows(dev):
         assert np.array_equal(cand[r], ri[r]) and np.array_equal(vals[r], rv[r])
     assert np.array_equal(vals[1], [-np.inf, -np.inf])
     assert cand[2, 0] == 77 and vals[2, 0] == np.inf
+
+
+@pytest.mark.parametrize("dtype,few,many", [(torch.bfloat16, (1, 2), (3, 5, 16, 17, 33)), (torch.float16, (1, 2), (3, 17)),
+                                            (torch.float32, (1, 2, 4), (5, 16, 21))])
+def test_head_rows_do_not_depend_on_the_batch_within_a_kernel(dev, dtype, few, many):
+    """A row's logits are the same bits in every call of few rows, and in every call of more; the
+    rerank of given candidates is the same in all."""
+    from mrun_pub_amd import qrow as q
+
+    v, k = 4099, 1536
+    g = torch.Generator(device=dev).manual_seed(4)
+    codes = torch.randint(-127, 128, (v, k), dtype=torch.int8, device=dev, generator=g)
+    scales = torch.rand(v, device=dev, generator=g) + 0.5
+    x = torch.randn(max(many), k, device=dev, generator=g).to(dtype)
+    page = q.CompactQRowPage("h", 0, v, k, codes, scales)
+    for sizes in (few, many):
+        ref = q.fused_qrow_top2(page, x[:sizes[-1]])
+        for m in sizes[:-1]:
+            got = q.fused_qrow_top2(page, x[:m])
+            assert torch.equal(got[0], ref[0][:m]) and torch.equal(got[1], ref[1][:m])
+    cand = q.fused_qrow_top2(page, x)[0]
+    best, score = q.rerank_qrow_candidates_fp32(page, x, cand)
+    for m in few + many:
+        b, s = q.rerank_qrow_candidates_fp32(page, x[:m], cand[:m])
+        assert torch.equal(b, best[:m]) and torch.equal(s, score[:m])
