@@ -379,6 +379,11 @@ int qs_lowbit_dequant(const uint8_t* packed, int64_t row_bytes, const void* scal
  * split activations (F32), and with the bytes of a single row they still run, in more launches. */
 size_t qs_lowbit_workspace_bytes(int x_dtype, int64_t M, int64_t N, int64_t K, int group_size);
 
+/* The tile of a call of more than 16 BF16 or 5 F32 rows with that workspace, groups of 64 or
+ * 128 (host only): tile[0] the activation rows of a tile (an F32 row counts as three), tile[1]
+ * its K slices, tile[2] the activation rows of a launch.  QS_ERR_UNSUPPORTED for fewer rows. */
+int qs_lowbit_many_plan(int x_dtype, int64_t M, int64_t N, int64_t K, int group_size, int32_t* tile);
+
 /* Replaces QStoreInt3.matmul / QStoreInt2.matmul (qstore.py:1318-1341, 1451-1474):
  * y[m,n] = sum_k x[m,k] * w[n,k] in fp32, y F32 [M, N].  x BF16 or F32; bits 2 or 3; any
  * group size and K (the tiled kernels take G 64 / 128 with whole groups and 4-byte aligned

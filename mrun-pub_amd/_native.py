@@ -84,6 +84,7 @@ SIGNATURES: dict[str, tuple] = {
     "qs_moe_route_reduce_to": (_I, [_P, _I, _P, _P, _L, _I, _L, _P, _I, _P]),
     "qs_lowbit_dequant": (_I, [_P, _L, _P, _I, _P, _I, ctypes.c_float, _I, _I, _P, _L, _L, _P]),
     "qs_lowbit_workspace_bytes": (ctypes.c_size_t, [_I, _L, _L, _L, _I]),
+    "qs_lowbit_many_plan": (_I, [_I, _L, _L, _L, _I, _P]),
     "qs_lowbit_gemv": (_I, [_P, _I, _L, _P, _L, _P, _I, _P, _I, ctypes.c_float, _I, _I, _P, _L, _L, _L, _L, _P, ctypes.c_size_t, _P]),
     "qs_pager_create": (_I, [_P, ctypes.c_size_t, _I, ctypes.c_size_t, ctypes.POINTER(_P)]),
     "qs_pager_destroy": (_I, [_P]),

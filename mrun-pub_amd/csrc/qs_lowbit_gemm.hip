@@ -464,3 +464,18 @@ int run_lowbit_gemm(const LowbitGemm& a, void* workspace, size_t workspace_bytes
 }
 
 }  // namespace qs
+
+using namespace qs;
+
+extern "C" int qs_lowbit_many_plan(int x_dtype, int64_t M, int64_t N, int64_t K, int group_size, int32_t* tile) {
+  const bool f32 = x_dtype == QS_F32;
+  if (!tile || N < 1 || K < 1) return fail(QS_ERR_INVALID, "lowbit_many_plan: bad arguments");
+  if (M <= (f32 ? 5 : 16) || (group_size != 64 && group_size != 128))
+    return fail(QS_ERR_UNSUPPORTED, "lowbit_many_plan: more than 16 BF16 or 5 F32 rows, groups of 64 or 128");
+  const int64_t chunk = std::min(M, lg_chunk_rows(f32, N, K));
+  const LgPlan plan = lg_plan((f32 ? 3 : 1) * chunk, N, K, group_size, kLgMaxPart);
+  tile[0] = 16 * plan.MT;
+  tile[1] = plan.S;
+  tile[2] = (int32_t)std::min<int64_t>(chunk, INT_MAX);
+  return QS_OK;
+}

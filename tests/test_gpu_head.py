@@ -82,3 +82,27 @@ def test_head_rows_do_not_depend_on_the_batch_within_a_kernel(dev, dtype, few, m
     for m in few + many:
         b, s = q.rerank_qrow_candidates_fp32(page, x[:m], cand[:m])
         assert torch.equal(b, best[:m]) and torch.equal(s, score[:m])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_head_top2_of_wider_rows(dev, dtype):
+    """Activation rows inside wider ones: what lies past k is not read."""
+    import mrun_pub_amd._native as nat
+
+    v, k, m, ldx = 300, 640, 19, 640 + 16
+    rng = np.random.default_rng(8)
+    codes = rng.integers(-127, 128, size=(v, k), dtype=np.int8)
+    scales = np.full(v, 2.0 ** -6, np.float32)
+    x = (rng.integers(-8, 9, size=(m, k)) / 16.0).astype(np.float32)
+    xd = torch.full((m, ldx), float("nan"), dtype=dtype, device=dev)
+    xd[:, :k] = torch.from_numpy(x).to(dev).to(dtype)
+    c, s = torch.from_numpy(codes).to(dev), torch.from_numpy(scales).to(dev)
+    cand = torch.empty((m, 2), dtype=torch.int32, device=dev)
+    vals = torch.empty((m, 2), device=dev)
+    wsb = int(nat.load().qs_qrow_top2_workspace_bytes(m, v))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    nat.call("qs_qrow_top2", xd.data_ptr(), nat.dtype_code(dtype), ldx, c.data_ptr(), s.data_ptr(), m, v, k, 0,
+             ws.data_ptr(), wsb, cand.data_ptr(), vals.data_ptr(), nat.stream_of(dev))
+    ri, rv = oq.qrow_top2(oq.head_logits(codes, scales, x, "bf16" if dtype == torch.bfloat16 else "fp32"))
+    assert np.array_equal(cand.cpu().numpy(), ri)
+    assert np.array_equal(vals.cpu().numpy(), rv)

@@ -107,3 +107,44 @@ def test_many_fp32_rows_of_a_wide_block(dev):
     want = ref(x)
     for rows in (slice(0, 319), slice(319, 330)):
         assert oq.rel_l2(y[rows], want[rows]) <= TOL
+
+
+# The 64-row tiles, in one K slice and in several, with ragged rows and columns: input rows
+# wider than k (not read past it), output rows wider than n (not written past it).
+@pytest.mark.parametrize("bits", [2, 3])
+@pytest.mark.parametrize("G,asym", [(64, True), (64, False), (128, True), (128, False)])
+@pytest.mark.parametrize("dt,m,n,k,split", [
+    (torch.bfloat16, 131, 4093, 128, False), (torch.bfloat16, 33, 11007, 256, False),
+    (torch.bfloat16, 33, 4093, 4096, True), (torch.bfloat16, 131, 4093, 11008, True),
+    (torch.float32, 65, 4093, 128, False), (torch.float32, 33, 2049, 4096, True)])
+def test_many_rows_64_row_tiles(dev, bits, G, asym, dt, m, n, k, split):
+    import mrun_pub_amd._native as nat
+
+    tile = (nat.ctypes.c_int32 * 4)()
+    xdt = nat.dtype_code(dt)
+    assert nat.load().qs_lowbit_many_plan(xdt, m, n, k, G, tile) == 0
+    assert tile[0] == 64 and (tile[1] > 1) == split  # another size for this tile if this fails
+    g = torch.Generator(device=dev).manual_seed(m + n + k + bits)
+    codes = torch.randint(0, 1 << bits, (n, k), dtype=torch.uint8, device=dev, generator=g)
+    words = sum(codes.view(n, k // 8, 8)[:, :, i].to(torch.int32) << (bits * i) for i in range(8))
+    packed = torch.stack([(words >> (8 * b)) & 255 for b in range(bits)], dim=2).to(torch.uint8).reshape(n, -1)
+    ng = k // G
+    scales = (torch.rand(n, ng, device=dev, generator=g) + 0.5) / 8
+    offset = 4.0 if bits == 3 else 1.0
+    zeros = None
+    if asym:
+        scales, zeros = scales.half(), (offset + 0.5 * torch.randn(n, ng, device=dev, generator=g)).half()
+    z = zeros.double() if asym else torch.full((n, ng), offset, dtype=torch.float64, device=dev)
+    w = ((codes.double().view(n, ng, G) - z[:, :, None]) * scales.double()[:, :, None]).view(n, k)
+    ldx, ldy = k + 64, n + 3
+    x = torch.full((m, ldx), float("nan"), dtype=dt, device=dev)
+    x[:, :k] = torch.randn(m, k, device=dev, generator=g).to(dt)
+    y = torch.full((m, ldy), 7.0, device=dev)
+    wsb = int(nat.load().qs_lowbit_workspace_bytes(xdt, m, n, k, G))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    nat.call("qs_lowbit_gemv", x.data_ptr(), xdt, ldx, packed.data_ptr(), packed.shape[1], scales.data_ptr(),
+             nat.dtype_code(scales.dtype), nat.ptr(zeros), nat.QS_F16 if asym else nat.QS_F32, offset, bits, G,
+             y.data_ptr(), ldy, m, n, k, ws.data_ptr(), wsb, nat.stream_of(dev))
+    want = x[:, :k].double() @ w.t()
+    assert float((y[:, :n].double() - want).norm() / want.norm()) <= TOL
+    assert bool((y[:, n:] == 7.0).all())

@@ -246,6 +246,33 @@ def test_prefill_ragged_widths_split(dev, dt, m, ns, k, swiglu, vec):
     assert _check_entry(dev, dt, m, ns, k, swiglu=swiglu, pad=pad, split=False) == 0
 
 
+# Every tile shape, (activation rows, K parts) with one slice and with several, which the sizes
+# above reach only in part: ragged rows and columns, wider input rows (not read past k), wider
+# output rows (not written past n) that allow vector stores and that start off alignment.
+@pytest.mark.parametrize("dt,swiglu,m,n,k,tile,split", [
+    (torch.bfloat16, False, 37, 301, 128, (32, 2), False), (torch.bfloat16, False, 37, 1030, 2048, (32, 2), True),
+    (torch.bfloat16, False, 1029, 1030, 128, (64, 2), False), (torch.bfloat16, False, 777, 37, 4096, (64, 2), True),
+    (torch.bfloat16, False, 300, 1030, 64, (128, 1), False), (torch.bfloat16, False, 65, 4099, 4096, (128, 1), True),
+    (torch.bfloat16, False, 200, 8961, 1536, (128, 2), False), (torch.bfloat16, False, 389, 1537, 4096, (128, 2), True),
+    (torch.float16, False, 1029, 1030, 128, (64, 2), False), (torch.float16, False, 65, 4099, 4096, (128, 1), True),
+    (torch.float16, False, 200, 8961, 1536, (128, 2), False), (torch.float16, False, 389, 1537, 4096, (128, 2), True),
+    (torch.bfloat16, True, 37, 301, 128, (32, 2), False), (torch.bfloat16, True, 37, 301, 2048, (32, 2), True),
+    (torch.bfloat16, True, 33, 8961, 128, (64, 2), False), (torch.bfloat16, True, 33, 1030, 4096, (64, 2), True),
+    (torch.bfloat16, True, 129, 777, 64, (128, 1), False), (torch.bfloat16, True, 65, 2049, 4096, (128, 1), True),
+    (torch.bfloat16, True, 65, 8961, 1536, (128, 2), False), (torch.bfloat16, True, 389, 777, 4096, (128, 2), True),
+    (torch.float32, False, 37, 301, 128, (16, 2), False), (torch.float32, False, 37, 301, 1536, (16, 2), True),
+    (torch.float32, False, 515, 1537, 320, (32, 2), False), (torch.float32, False, 149, 130, 8960, (32, 2), True)])
+@pytest.mark.parametrize("layout", ["packed", "wide", "misaligned"])
+def test_prefill_every_tile_and_layout(dev, dt, swiglu, m, n, k, tile, split, layout):
+    from mrun_pub_amd import qrow as q
+
+    plan = (q.nat.ctypes.c_int32 * 4)()
+    q.nat.load().qs_qrow_prefill_plan(q.nat.dtype_code(dt), m, 1, q.nat.int64_array([n]), k, int(swiglu), int(split), plan)
+    assert (plan[0], plan[2]) == tile and (plan[3] > 1) == split  # another size for this tile if this fails
+    kw = {"packed": {}, "wide": dict(ldx=k + 64, pad=8 - n % 4), "misaligned": dict(ldx=k + 8, pad=-n % 4, shift=1)}[layout]
+    assert (_check_entry(dev, dt, m, [n], k, swiglu=swiglu, split=split, **kw) > 0) == split
+
+
 def test_prefill_rows_past_one_launch(dev):
     """More rows than one grid's 2^32 threads hold: 32-row tiles of one column reach that at 2^28
     rows (a 69 GB input).  All rows are zero but a few on both sides of every edge."""
