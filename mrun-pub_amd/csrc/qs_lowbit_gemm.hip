@@ -1,7 +1,7 @@
 // Packed int3 / int2 products of many activation rows on gfx950.
 //
 //   k_lowbit_gemm    y[m, n] = sum_k x[m, k] w[n, k] for a tile of 16 * MT bf16 rows and
-//                    64 * NT weight rows x one K slice, the formula of k_lowbit_gk per group
+//                    64 weight rows x one K slice, the formula of k_lowbit_gk per group
 //   k_lowbit_sum     the slices' (and, for fp32 activations, the three bf16 terms') partial
 //                    sums added in order
 #include "qs_lowbit.h"
@@ -47,19 +47,21 @@ __device__ __forceinline__ void lg_wait_barrier() {
 }
 
 // What bounds it: per group and 16 x 16 tile, 2 or 4 MFMAs (as many again per 16 activation
-// rows for the group sums, shared by NT row blocks), 8 VALU operations to apply the zero point
-// and the scale in fp32 (the weights are fp32: folding the scale into the bf16 operand would
-// round them), the unpacking of the wave's codes (19 VALU operations per 16 int2 codes, 24 per
-// 16 int3) and the scale gathers; no single one dominates.  Activations reach LDS by DMA in
-// 128-k steps shared by four waves, codes and scales go global -> VGPR, both two steps ahead.
-// k_lowbit_gk, one launch per 16 rows, reads and unpacks all codes for each of them.  Measured
-// (start of both: k_lowbit_gk): int2 G = 128 131 x 4096 x 11008 124 -> 38 us, int3 G = 64
-// 131 x 11008 x 4096 110 -> 60, 393 x 4096 x 11008 360 -> 109, 17 rows 26 -> 21 / 29 -> 17.
-// A step's two G = 64 scales (and zero points) in one load each: 74 -> 60 us at 131 rows.
-template <int BITS, int G, int SZ, int MT, int NT>
+// rows for the group sums), 8 VALU operations to apply the zero point and the scale in fp32
+// (the weights are fp32: folding the scale into the bf16 operand would round them), the
+// unpacking of the wave's codes (19 VALU operations per 16 int2 codes, 24 per 16 int3) and the
+// scale gathers; no single one dominates (by counter, 131 rows: the matrix pipe is busy 36% of
+// the time at G = 128 and 22% at G = 64, half of it with the group sums; LDS reads take 37% at
+// G = 128, half of it bank conflicts).  Activations reach LDS by DMA in 128-k steps shared by
+// four waves, codes and scales go global -> VGPR, both two steps ahead.  k_lowbit_gk, one launch
+// per 16 rows, reads and unpacks all codes for each of them.  Measured against it: int2 G = 128
+// 131 x 4096 x 11008 124 -> 38 us, int3 G = 64 131 x 11008 x 4096 110 -> 60,
+// 393 x 4096 x 11008 360 -> 109, 17 rows 26 -> 21 / 29 -> 17.  A step's two G = 64 scales (and
+// zero points) in one load each: 74 -> 60 us at 131 rows.
+template <int BITS, int G, int SZ, int MT>
 __global__ __launch_bounds__(256, 2) void k_lowbit_gemm(LgParams p) {
   constexpr float OFF = BITS == 3 ? 8.f : 0.f;
-  constexpr int TM = 16 * MT, TN = 64 * NT;
+  constexpr int TM = 16 * MT, TN = 64;
   constexpr int D = 2;             // steps in flight
   constexpr int GPS = 128 / G;     // groups per step
   constexpr int NJ = G / 32;       // MFMAs per group
@@ -70,7 +72,7 @@ __global__ __launch_bounds__(256, 2) void k_lowbit_gemm(LgParams p) {
   constexpr int XD = MT;           // 1 KiB copies per wave per stage
   constexpr int SW = GPS * (SZ ? 2 : 4) / 4 > 0 ? GPS * (SZ ? 2 : 4) / 4 : 1;  // scale words per step
   constexpr bool PAIR = GPS == 2;  // a step's two groups: their scales are loaded together
-  constexpr int GROUP = XD + NT * (GPS + (SZ ? 2 : 1));
+  constexpr int GROUP = XD + GPS + (SZ ? 2 : 1);
   __shared__ __attribute__((aligned(1024))) uint8_t lds[(D + 1) * STAGE];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -124,44 +126,41 @@ __global__ __launch_bounds__(256, 2) void k_lowbit_gemm(LgParams p) {
     for (int e = 0; e < XD; ++e)
       lg_copy16(xr, lds + st * STAGE + xdst[e], xk[e] < room ? xoff[e] : xlim, i < T ? k0 * 2 : 0);
   };
-  uint32_t cw[D][NT][GPS][NWD];
-  uint32_t sw[D][NT][SW], zw[D][NT][SW];
+  uint32_t cw[D][GPS][NWD];
+  uint32_t sw[D][SW], zw[D][SW];
   const int qoff = BITS == 3 && G == 64 ? (6 * q) & ~3 : QB * q;
   auto load_w = [&](int b, int i) {
+    const int r = 16 * wave + col;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int r = 16 * (NT * wave + j) + col;
-#pragma unroll
-      for (int gi = 0; gi < GPS; ++gi) {
-        const int g = (t0 + i) * GPS + gi;
-        const bool live = i < T && g < ng;
-        const int wo = live ? r * (int)p.row_bytes + g * CB + qoff : wlim;
-        if constexpr (NWD == 1) {
-          cw[b][j][gi][0] = __builtin_amdgcn_raw_buffer_load_b32(wr, wo, 0, 0);
-        } else if constexpr (NWD == 2) {
-          const auto v = __builtin_amdgcn_raw_buffer_load_b64(wr, wo, 0, 0);
-          cw[b][j][gi][0] = v[0];
-          cw[b][j][gi][1] = v[1];
-        } else {
-          const auto v = __builtin_amdgcn_raw_buffer_load_b96(wr, wo, 0, 0);
-          cw[b][j][gi][0] = v[0];
-          cw[b][j][gi][1] = v[1];
-          cw[b][j][gi][2] = v[2];
-        }
-      }
-      // (an even group count keeps both groups of a step on one side of the row's end)
-      const int g = (t0 + i) * GPS;
-      const int so = i < T && g < ng ? (r * ng + g) * ES : slim;
-      if constexpr (SZ) {
-        sw[b][j][0] = PAIR ? __builtin_amdgcn_raw_buffer_load_b32(sr, so, 0, 0) : __builtin_amdgcn_raw_buffer_load_b16(sr, so, 0, 0);
-        zw[b][j][0] = PAIR ? __builtin_amdgcn_raw_buffer_load_b32(zr, so, 0, 0) : __builtin_amdgcn_raw_buffer_load_b16(zr, so, 0, 0);
-      } else if constexpr (PAIR) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(sr, so, 0, 0);
-        sw[b][j][0] = v[0];
-        sw[b][j][1] = v[1];
+    for (int gi = 0; gi < GPS; ++gi) {
+      const int g = (t0 + i) * GPS + gi;
+      const bool live = i < T && g < ng;
+      const int wo = live ? r * (int)p.row_bytes + g * CB + qoff : wlim;
+      if constexpr (NWD == 1) {
+        cw[b][gi][0] = __builtin_amdgcn_raw_buffer_load_b32(wr, wo, 0, 0);
+      } else if constexpr (NWD == 2) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(wr, wo, 0, 0);
+        cw[b][gi][0] = v[0];
+        cw[b][gi][1] = v[1];
       } else {
-        sw[b][j][0] = __builtin_amdgcn_raw_buffer_load_b32(sr, so, 0, 0);
+        const auto v = __builtin_amdgcn_raw_buffer_load_b96(wr, wo, 0, 0);
+        cw[b][gi][0] = v[0];
+        cw[b][gi][1] = v[1];
+        cw[b][gi][2] = v[2];
       }
+    }
+    // (an even group count keeps both groups of a step on one side of the row's end)
+    const int g = (t0 + i) * GPS;
+    const int so = i < T && g < ng ? (r * ng + g) * ES : slim;
+    if constexpr (SZ) {
+      sw[b][0] = PAIR ? __builtin_amdgcn_raw_buffer_load_b32(sr, so, 0, 0) : __builtin_amdgcn_raw_buffer_load_b16(sr, so, 0, 0);
+      zw[b][0] = PAIR ? __builtin_amdgcn_raw_buffer_load_b32(zr, so, 0, 0) : __builtin_amdgcn_raw_buffer_load_b16(zr, so, 0, 0);
+    } else if constexpr (PAIR) {
+      const auto v = __builtin_amdgcn_raw_buffer_load_b64(sr, so, 0, 0);
+      sw[b][0] = v[0];
+      sw[b][1] = v[1];
+    } else {
+      sw[b][0] = __builtin_amdgcn_raw_buffer_load_b32(sr, so, 0, 0);
     }
   };
 
@@ -206,25 +205,18 @@ __global__ __launch_bounds__(256, 2) void k_lowbit_gemm(LgParams p) {
   };
 
   const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-  f32x4 y[NT][MT], sum[NT][MT];
+  f32x4 y[MT], sum[MT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int m = 0; m < MT; ++m) y[j][m] = sum[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < MT; ++m) y[m] = sum[m] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto mul = [&](int b, int i, int st) {
     const uint8_t* xs = lds + st * STAGE + col * 256;
 #pragma unroll
     for (int gi = 0; gi < GPS; ++gi) {
-      u32x4 f[NT][NJ];
+      u32x4 f[NJ];
+      unpack(cw[b][gi], f);
+      f32x4 s0[MT], d[MT];
 #pragma unroll
-      for (int j = 0; j < NT; ++j) unpack(cw[b][j][gi], f[j]);
-      f32x4 s0[MT], d[NT][MT];
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        s0[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < NT; ++j) d[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+      for (int m = 0; m < MT; ++m) s0[m] = d[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int e = 0; e < NJ; ++e) {
         const int ch = (G == 64 ? 8 * gi + 2 * q : 4 * q) + e;
@@ -232,20 +224,15 @@ __global__ __launch_bounds__(256, 2) void k_lowbit_gemm(LgParams p) {
         for (int m = 0; m < MT; ++m) {
           const bf16x8 x = *reinterpret_cast<const bf16x8*>(xs + 4096 * m + 16 * (ch ^ col));
           s0[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, ones, s0[m], 0, 0, 0);
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-            d[j][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(bf16x8, f[j][e]), d[j][m], 0, 0, 0);
+          d[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(bf16x8, f[e]), d[m], 0, 0, 0);
         }
       }
+      const float sc = SZ ? f16_bits_to_f32((uint16_t)(sw[b][0] >> (16 * gi))) : __uint_as_float(sw[b][gi % SW]);
+      const float cz = OFF + (SZ ? f16_bits_to_f32((uint16_t)(zw[b][0] >> (16 * gi))) : p.offset);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const float sc = SZ ? f16_bits_to_f32((uint16_t)(sw[b][j][0] >> (16 * gi))) : __uint_as_float(sw[b][j][gi % SW]);
-        const float cz = OFF + (SZ ? f16_bits_to_f32((uint16_t)(zw[b][j][0] >> (16 * gi))) : p.offset);
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) y[j][m][r] = fmaf(sc, fmaf(-cz, s0[m][r], d[j][m][r]), y[j][m][r]);
-      }
+        for (int r = 0; r < 4; ++r) y[m][r] = fmaf(sc, fmaf(-cz, s0[m][r], d[m][r]), y[m][r]);
     }
     load_w(b, i + D);
   };
@@ -270,12 +257,10 @@ __global__ __launch_bounds__(256, 2) void k_lowbit_gemm(LgParams p) {
   // 1.1e-7 of 64-bit sums)
   auto flush = [&]() {
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        sum[j][m] += y[j][m];
-        y[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+    for (int m = 0; m < MT; ++m) {
+      sum[m] += y[m];
+      y[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
   };
   for (int i = 0;;) {  // the loop's shape keeps the load counts exact (see k_prefill)
     step(0, i);
@@ -293,18 +278,15 @@ __global__ __launch_bounds__(256, 2) void k_lowbit_gemm(LgParams p) {
 
   // lane holds D[m = 4 q + r][n = col] of each tile
   float* out = p.out + (int64_t)s * p.M * p.ldo;
+  const int n = tb + 16 * wave + col;
+  if (n >= p.N) return;
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int n = tb + 16 * (NT * wave + j) + col;
-    if (n >= p.N) continue;
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = bm + 16 * m + 4 * q + r;
-        if (row < p.M) out[(int64_t)row * p.ldo + n] = sum[j][m][r];
-      }
-  }
+    for (int r = 0; r < 4; ++r) {
+      const int row = bm + 16 * m + 4 * q + r;
+      if (row < p.M) out[(int64_t)row * p.ldo + n] = sum[m][r];
+    }
 }
 
 // y[m, n] = sum over the rpx terms of row m of the sum over slices s of part[s][rpx m + t][n]
@@ -370,8 +352,8 @@ LgPlan lg_plan(int64_t rows, int64_t N, int64_t K, int G, int64_t part_cap) {
 template <int BITS, int G, int SZ>
 void lg_launch(const LgParams& p, int mt, hipStream_t s) {
   const dim3 grid((unsigned)((int64_t)p.tiles_m * p.tiles_n * p.S));
-  if (mt == 2) hipLaunchKernelGGL((k_lowbit_gemm<BITS, G, SZ, 2, 1>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((k_lowbit_gemm<BITS, G, SZ, 4, 1>), grid, dim3(256), 0, s, p);
+  if (mt == 2) hipLaunchKernelGGL((k_lowbit_gemm<BITS, G, SZ, 2>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((k_lowbit_gemm<BITS, G, SZ, 4>), grid, dim3(256), 0, s, p);
 }
 
 // Activation rows per launch.  fp32 (three bf16 rows each): at most 512, and no more than keep

@@ -60,31 +60,32 @@ __device__ __forceinline__ void pf_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// A wave's accumulators go to separate sums every kPfFlush of its 64-k steps (12 MFMAs): one
+// A wave's accumulators go to separate sums every six of its 64-k steps (12 MFMAs): one
 // fp32 chain over a whole row of 1536..8960 k would be less exact than the short chains of
 // the batched kernels' K splits (outputs of 1531 x 1536 x 8960 that round differently from
 // the exact sum: rel-L2 4.7e-5 in one chain, 1.8e-5 with the flushes, 1.9e-5 batched; they
 // cost 2-3% of the time).
-constexpr int kPfFlush = 6;
-
+//
 // What bounds it and why this split: the dequantized weight element costs 2.5 VALU operations,
 // so it is made once per 16 * MT activation rows, in the registers of the one wave (of its
 // K part) that owns the weight row: weights go global -> VGPR, and only activations pass
-// through LDS, copied by DMA and read by all WN waves.  At MT = 8 the conversion takes 62% of
-// the time of the MFMAs it feeds and the LDS reads half of the LDS rate.  Measured (1531 rows,
+// through LDS, copied by DMA and read by all WN waves.  Measured in graph replays (1531 rows,
 // one launch, before: 32-row batches of the batched kernel): paired SwiGLU 8960 x 1536
-// 558 -> 104 us (810 TFLOP/s), 1536 x 8960 521 -> 67 us, q/k/v 241 -> 19 us.  Timing probes of
-// the 128-row tile on one box, 114 us whole: no conversion 101, no LDS reads 103, no copies
-// 100, no weight loads 105, MFMAs and epilogue alone 63: no single phase bounds it, the
-// phases of a CU's two or three workgroups overlap only in part.  Pinning the conversions
-// between the MFMAs (one pair of codes per two MFMAs) was 10% slower, as was a third group in
-// flight.
+// 497 -> 113 us (745 TFLOP/s; traced 113 to 124 on several cards), 1536 x 8960 481 -> 70 us
+// with its reduce, 1536 x 1536 213 -> 20 us.  At MT = 8 the loop's conversion instructions
+// take 62% of the issue time of the MFMAs they feed, the other VALU ones 22%; the matrix pipe
+// is busy 32% of the SwiGLU's time by counter, and LDS reads 33%, half of those cycles bank
+// conflicts.  Timing probes of the 128-row tile on one box, 114 us whole: no conversion 101, no
+// LDS reads 103, no copies 100, no weight loads 105, MFMAs and epilogue alone 63: no single
+// phase bounds it, the phases of a CU's two or three workgroups overlap only in part.  Pinning
+// the conversions between the MFMAs (one pair of codes per two MFMAs) was 10% slower, as was a
+// third group in flight.
 //
 // fp32 activations run on v_mfma_f32_16x16x4 (a sixteenth of the bf16 rate), so there the
 // matrix pipe is the bound and the tiles are small (16 or 32 rows) to keep every CU's busy:
-// 149 x 1536 x 8960 787 -> 54 us (75 TFLOP/s of the 135 that a 4096^3 library product reaches;
-// before: one launch of the one-row VALU kernel per row), 64 x 8960 x 1536 155 -> 29 us,
-// 9 x 4096 x 1024 15.0 -> 8.4 us.  Error against 64-bit sums 1.0e-7..1.2e-7 (VALU: 1.0e-7 at
+// 149 x 1536 x 8960 785 -> 54 us (75 TFLOP/s of the 135 that a 4096^3 library product reaches,
+// the pipe busy half of the time; before: one launch of the one-row VALU kernel per row),
+// 64 x 8960 x 1536 148 -> 29 us, 16 x 4096 x 1024 19.3 -> 8.8 us.  Error against 64-bit sums 1.0e-7..1.2e-7 (VALU: 1.0e-7 at
 // K = 1024 to 2.3e-7 at K = 8960).
 template <int P, int MT, int NT, int WN, int WK, int XT>
 __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
@@ -157,8 +158,8 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
         const_cast<int8_t*>(p.lin[P == 2 ? pl : li].codes + (int64_t)tb * K), (short)0, wlim, 0x00020000);
 
   // copy e of a stage: whole rows of one 64-k step; lane l lands in row l / SL, slot l % SL,
-  // which holds 16-byte chunk slot ^ (a hash of the row) (the 16 rows a fragment pass reads
-  // then fall in distinct bank groups)
+  // which holds 16-byte chunk slot ^ (a hash of the row): the 16 rows that 16 lanes of a
+  // fragment read touch fall in distinct bank groups
   auto swz = [](int r) { return F32 ? r & 15 : (r >> 1) & 7; };
   int xoff[XD], xsub[XD], xdst[XD];
 #pragma unroll
@@ -301,7 +302,6 @@ __global__ __launch_bounds__(WN * WK * 64, 2) void k_prefill(PfParams p) {
     mul(w[d], i, st);
     st = st == D ? 0 : st + 1;
   };
-  static_assert(kPfFlush == 6, "steps between flushes below");
   for (int i = 0;;) {
     step(0, i);
     if (++i >= I) break;
@@ -538,7 +538,7 @@ int64_t pf_launch_rows(const PfPlan& plan) {
 // Whether the prefill kernel is expected to beat the launches that qs_qrow_matmul_multi and
 // qs_qrow_swiglu otherwise make, from `split` or unsplit plan times against their times in
 // microseconds (graph replays, 2 to 512 rows of the shapes below and their K and N in other
-// pairs).  K that those kernels do not take runs one wave per weight row there: always prefill.
+// pairs).  Rows longer than those kernels take run one wave per weight row there: always prefill.
 bool prefill_faster(int x_dtype, int64_t M, int n_lin, const int64_t* N, int64_t K, int P, bool split) {
   if (M < 2) return false;
   float rows = 0.f;  // millions of weights

@@ -11,14 +11,15 @@
 //                                 multiply-add, so the VALU only pays for the dequant
 //                                 (cvt_sdwa + mul + half a cvt_pk per weight byte).
 //                                 K is split across the waves of a workgroup and reduced
-//                                 through LDS in a fixed order.  Used for 5 <= M.
+//                                 through LDS in a fixed order.  Used for 5 <= M <= 32,
+//                                 and for batches of 32 where k_prefill is slower.
 //   k_w8a16_s<...>              : the same contract as a streaming kernel -- one wave per
 //                                 (tile, K slice) with a sliding window of chunks in
 //                                 flight, SwiGLU planes sharing a wave, activations in LDS
 //                                 when they are small.  Used for SwiGLU at 5 <= M and for
 //                                 long rows (K >= 4096) while the activations fit in LDS.
-//   k_gemv_valu<...>            : M <= 4 bf16/f16 decode rows and every fp32-activation
-//                                 call: one wave per weight row, 1 KiB
+//   k_gemv_valu<...>            : M <= 4 bf16/f16 decode rows and few fp32 rows (more of
+//                                 either: k_prefill, k_bd2): one wave per weight row, 1 KiB
 //                                 contiguous row segments per instruction issued in row
 //                                 order through a 4-chunk window, exact-width tail,
 //                                 VALU dequant + fma / v_dot2, fixed-order DPP wave sum.
@@ -1918,6 +1919,8 @@ int run_linears(QrowParams p, int x_dtype, int64_t M, hipStream_t s, bool row_st
   if ((row_stable || M <= kValuRows || x_dtype == QS_F32) && valu_eligible(p, x_dtype))
     return run_valu(p, x_dtype, M, s, false);
   if (!row_stable && mfma_eligible(p, x_dtype)) {
+    // more than one batch: 33 to 64 rows that many_rows() leaves, or rows so far apart that
+    // k_prefill's 31-bit offsets do not reach them
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
       QrowParams q = p;
       const int mm = (int)((M - m0) < 32 ? (M - m0) : 32);
@@ -2083,6 +2086,8 @@ extern "C" int qs_qrow_swiglu(const void* x, int64_t ldx, const int8_t* gate_cod
     if (st != QS_ERR_UNSUPPORTED) return st;
   }
   if (mfma_eligible(p, QS_BF16)) {
+    // more than one batch: rows so far apart (4 M elements) that k_prefill's 31-bit offsets do
+    // not reach them
     for (int64_t m0 = 0; m0 < M; m0 += 32) {
       QrowParams q = p;
       const int mm = (int)((M - m0) < 32 ? (M - m0) : 32);
