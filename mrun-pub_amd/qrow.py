@@ -207,30 +207,30 @@ def _prefill_eligible(x2: torch.Tensor, codes: list[torch.Tensor], swiglu: bool 
 def _run_batched(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
                  swiglu: bool) -> None:
     """At most 32 16-bit rows through the batched kernels (the split depends on N and K only)."""
+    m, k = x2.shape
     ns = nat.int64_array([int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]])
-    _run_many("batched", x2, pages, outs, swiglu, ns,
-              int(nat.load().qs_qrow_batched_workspace_bytes(x2.shape[0], len(ns), ns, x2.shape[1], int(swiglu))))
+    _run_many("batched", x2, m, k, pages, outs, swiglu, ns,
+              nat.load().qs_qrow_batched_workspace_bytes(m, len(ns), ns, k, swiglu))
 
 
 def _run_prefill(x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
                  swiglu: bool) -> bool:
     """Any number of rows through the prefill kernel; ``False``, with nothing launched, where
     the kernels of the plain entry points are expected to be faster."""
+    m, k = x2.shape
     ns = nat.int64_array([int(c.shape[0]) for c, _ in pages[:1 if swiglu else len(pages)]])
-    ws_bytes = int(nat.load().qs_qrow_prefill_plan(nat.dtype_code(x2.dtype), x2.shape[0], len(ns), ns, x2.shape[1],
-                                                   int(swiglu), 1, None))
+    ws_bytes = nat.load().qs_qrow_prefill_plan(nat.dtype_code(x2.dtype), m, len(ns), ns, k, swiglu, 1, None)
     if ws_bytes < 0:
         return False
-    _run_many("prefill", x2, pages, outs, swiglu, ns, ws_bytes)
+    _run_many("prefill", x2, m, k, pages, outs, swiglu, ns, ws_bytes)
     return True
 
 
-def _run_many(kind: str, x2: torch.Tensor, pages: list[tuple[torch.Tensor, torch.Tensor]], outs: list[torch.Tensor],
-              swiglu: bool, ns, ws_bytes: int) -> None:
+def _run_many(kind: str, x2: torch.Tensor, m: int, k: int, pages: list[tuple[torch.Tensor, torch.Tensor]],
+              outs: list[torch.Tensor], swiglu: bool, ns, ws_bytes: int) -> None:
     """``qs_qrow_matmul_<kind>`` / ``qs_qrow_swiglu_<kind>`` with a workspace for the K-slice
     partial sums."""
     device = x2.device
-    m, k = int(x2.shape[0]), int(x2.shape[1])
     stream = nat.stream_of(device)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
     if swiglu:
