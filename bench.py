@@ -445,6 +445,65 @@ def profile_lowbit(torch, dev, calls: int) -> dict:
     return out
 
 
+def profile_many_rows(torch, dev, calls: int) -> dict:
+    """Eager launches of the many-row products, ``calls`` each on two weight sets in turn: the
+    linears of a bf16 1536 / 8960 layer for 1531 rows, an fp32 1536 x 8960 one for 149, the
+    top-2 search of a 151,936 x 1536 head for 11 bf16 and fp32 rows, packed int2 (G 128, fixed
+    offset) and int3 (G 64, zero points) linears for 131 rows; prints each one's algorithmic
+    bytes and operations."""
+    from mrun_pub_amd import lowbit, qrow
+
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(3)
+    out: dict = {"profile": "many", "calls": calls}
+
+    def weights(n, k):
+        return [qrow.CompactQRowPage("w", 0, n, k, torch.randint(-127, 128, (n, k), dtype=torch.int8, device=dev,
+                                                                 generator=gen),
+                                     (torch.rand(n, device=dev, generator=gen) + 0.5) / (73 * k ** 0.5)) for _ in range(2)]
+
+    def rows(m, k, dt):
+        return torch.randn(m, k, device=dev, generator=gen).to(dt)
+
+    def case(name, fn, read, written, ops):
+        for i in range(calls):
+            fn(i % 2)
+        out[name] = {"read_bytes": read, "written_bytes": written, "ops": ops}
+
+    bf, m, h, kv, inter = torch.bfloat16, 1531, 1536, 256, 8960
+    q, k, v, o, g, u, d = (weights(*s) for s in ((h, h), (kv, h), (kv, h), (h, h), (inter, h), (inter, h), (h, inter)))
+    x, act = rows(m, h, bf), rows(m, inter, bf)
+    n = h + 2 * kv
+    case("qkv", lambda i: qrow.qrow_matmul_multi([(p[i].codes, p[i].scales) for p in (q, k, v)], x),
+         n * (h + 4) + 2 * m * h, 2 * m * n, 2 * m * n * h)
+    case("o", lambda i: qrow.qrow_matmul(o[i].codes, o[i].scales, x), h * (h + 4) + 2 * m * h, 2 * m * h, 2 * m * h * h)
+    case("swiglu", lambda i: qrow.fused_qrow_swiglu(g[i], u[i], x), 2 * inter * (h + 4) + 2 * m * h, 2 * m * inter,
+         4 * m * inter * h)
+    case("down", lambda i: qrow.qrow_matmul(d[i].codes, d[i].scales, act), h * (inter + 4) + 2 * m * inter, 2 * m * h,
+         2 * m * h * inter)
+    xf = rows(149, inter, torch.float32)
+    case("f32", lambda i: qrow.qrow_matmul(d[i].codes, d[i].scales, xf), h * (inter + 4) + 4 * 149 * inter, 4 * 149 * h,
+         2 * 149 * h * inter)
+    head = weights(151936, h)
+    for dt, es in ((bf, 2), (torch.float32, 4)):
+        xh = rows(11, h, dt)
+        case(f"head_{str(dt)[6:]}", lambda i: qrow.fused_qrow_top2(head[i], xh), 151936 * (h + 4) + es * 11 * h, 11 * 16,
+             2 * 11 * 151936 * h)
+    for bits, G, N, K in ((2, 128, 4096, 11008), (3, 64, 11008, 4096)):
+        rb, ng = K * bits // 8, K // G
+        pages = []
+        for _ in range(2):
+            packed = torch.randint(0, 256, (N, rb), dtype=torch.uint8, device=dev, generator=gen)
+            sc = (torch.rand(N, ng, device=dev, generator=gen) + 0.5) / 7
+            zp = (torch.rand(N, ng, device=dev, generator=gen) * 7).half() if G == 64 else None
+            pages.append(lowbit.LowbitPage("w", bits, G, K, packed, sc.half() if G == 64 else sc, zp))
+        xl = rows(131, K, bf)
+        case(f"int{bits}", lambda i: lowbit.lowbit_matmul(pages[i], xl), N * (rb + 4 * ng) + 2 * 131 * K, 4 * 131 * N,
+             2 * 131 * N * K)
+    torch.cuda.synchronize()
+    return out
+
+
 def profile_codecs(torch, dev, calls: int) -> dict:
     """Eager launches of the offline codecs, ``calls`` each: int8 rows of an fp32 [14336,
     4096] weight, int3 and int2 (G 128) of an fp32 [11008, 4096] one; prints each one's
@@ -752,14 +811,14 @@ def main() -> int:
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--cpu-seconds", type=float, default=6.0)
     ap.add_argument("--no-secondary", action="store_true", help="skip configs 1/3/4/5")
-    ap.add_argument("--profile", choices=("swiglu", "stack", "copy", "w8a8", "w8a8p", "moe", "moe16", "lowbit", "codec",
-                                          "dequant"),
+    ap.add_argument("--profile", choices=("swiglu", "stack", "copy", "w8a8", "w8a8p", "moe", "moe16", "lowbit", "many",
+                                          "codec", "dequant"),
                     help="for rocprofv3 runs: replay exactly the timed graph of the roofline kernel (28 "
                     "paired gate/up+SwiGLU launches) or of the headline pass, --steps times after "
                     "--warmup replays; a plain 256 MiB device copy x5 (counter calibration); or config 3's "
                     "fused W8A8 GEMM (M=512 and 2048), config 3's whole w8a8_matmul with protect_k=8 (w8a8p) / "
                     "config 4's MoE layer (T=64 and 512; moe16: the weight-only flow), or config 5's low-bit "
-                    "GEMV/GEMM (both shapes, int3/int2, M=1 and 8), the offline codecs (int8, int3, "
+                    "GEMV/GEMM (both shapes, int3/int2, M=1 and 8), the many-row (prefill) products, the offline codecs (int8, int3, "
                     "int2), or the whole-weight dequants (qrow bf16/fp32, int3/int2 fp32), --steps calls each")
     ap.add_argument("--eager", action="store_true",
                     help="with --profile swiglu/stack: launch the same sequence eagerly instead of replaying "
@@ -797,6 +856,9 @@ def main() -> int:
         return 0
     if args.profile == "lowbit":
         print(json.dumps(profile_lowbit(torch, dev, args.steps)), flush=True)
+        return 0
+    if args.profile == "many":
+        print(json.dumps(profile_many_rows(torch, dev, args.steps)), flush=True)
         return 0
     if args.profile == "codec":
         print(json.dumps(profile_codecs(torch, dev, args.steps)), flush=True)
