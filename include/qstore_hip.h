@@ -310,8 +310,10 @@ int qs_moe_gather_quant(const void* source, int src_dtype, int64_t ld_src, const
  * (F32/BF16); swiglu != 0: N_w = 2N, out[row, n] = bf16(bf16(silu(bf16(gate))) * bf16(up))
  * with gate from weight row n and up from row n + N.  K % 64 == 0, K <= 8192 with SwiGLU,
  * K <= 16384 without.  max_rows is the reference's max_rows argument
- * (qwen3_moe_cuda.py:2257-2310, callers pass the routed row count, :2747): a bound on
- * counts[g] used only to size the row tile (0 = unknown); results do not depend on it. */
+ * (qwen3_moe_cuda.py:2257-2310, callers pass the routed row count, :2747): the routed rows,
+ * or a bound on counts[g].  It only chooses the row tile and, below 2 G (int8) or 3 G (weight-
+ * only), smaller blocks dealt out over the groups that have rows, which a bound far below the
+ * routed rows makes up to 13% slower (0 = unknown); results do not depend on it. */
 int qs_moe_grouped_gemm_i8(const int8_t* a, const float* a_scale, const int8_t* w,
                            int64_t w_stride, const float* w_scale, int64_t ws_stride,
                            const int32_t* starts, const int32_t* counts, const int32_t* slots,

@@ -130,3 +130,15 @@ def test_lowbit_workspace_is_bounded(dtype, n, k):
     for m in (17, 149, 512, 4096, 100000):
         # partial sums and split rows, or what a single row takes
         assert size(getattr(nat, dtype), m, n, k, 64) <= max((256 + 64) << 20, one + 192 * k) + 512, m
+
+
+def test_rows_bound_of_the_grouped_products():
+    """A bound on one group's rows does not pass for a queue of few tokens, and keeps its row tile
+    (16 rows while the mean bound per group is at most 8)."""
+    from mrun_pub_amd.moe import _rows_bound
+
+    assert _rows_bound(None, 1024, 128) == 1024 and _rows_bound(0, 1024, 128) == 0
+    assert _rows_bound(4, 1024, 128) == 1024 and _rows_bound(4, 104, 128) == 104
+    assert _rows_bound(16, 6216, 128) == 8 * 128 and _rows_bound(4000, 1024, 128) == 4000
+    with pytest.raises(ValueError, match="non-negative"):
+        _rows_bound(-1, 8, 8)
