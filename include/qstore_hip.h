@@ -383,7 +383,9 @@ size_t qs_lowbit_workspace_bytes(int x_dtype, int64_t M, int64_t N, int64_t K, i
 
 /* The tile of a call of more than 16 BF16 or 5 F32 rows with that workspace, groups of 64 or
  * 128 (host only): tile[0] the activation rows of a tile (an F32 row counts as three), tile[1]
- * its K slices, tile[2] the activation rows of a launch.  QS_ERR_UNSUPPORTED for fewer rows. */
+ * its K slices, tile[2] the activation rows of a launch.  QS_ERR_UNSUPPORTED for fewer rows.
+ * (17 to 32 BF16 rows of some int2 widths run as two launches of 16 instead, and so do layouts
+ * that this kernel does not take.) */
 int qs_lowbit_many_plan(int x_dtype, int64_t M, int64_t N, int64_t K, int group_size, int32_t* tile);
 
 /* Replaces QStoreInt3.matmul / QStoreInt2.matmul (qstore.py:1318-1341, 1451-1474):

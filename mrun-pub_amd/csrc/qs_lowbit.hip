@@ -1210,10 +1210,23 @@ extern "C" int qs_lowbit_gemv(const void* x, int x_dtype, int64_t ldx, const uin
   if (!workspace || workspace_bytes < need)
     return fail(QS_ERR_INVALID, "lowbit_gemv: workspace of %zu bytes required", need);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // 3..16 bf16 rows take k_lowbit_gk.  Its scale / zero rows are read as 4-byte words (fp16
+  // arrays need an even group count), its code rows in 16-byte pieces.
+  const bool layout = (scale_dtype == QS_F16 && zeros && zero_dtype == QS_F16) || (scale_dtype == QS_F32 && !zeros);
+  const bool words = aligned(scales, 4) && (!zeros || aligned(zeros, 4)) && (scale_dtype == QS_F32 || ng % 2 == 0);
+  const int gk_waves = (int)cdiv(ng, group_size == 64 ? kGkGroupsLong<64> : kGkGroupsLong<128>);  // bounds every form
+  const bool gk_ok = x_dtype == QS_BF16 && layout && words && gk_waves <= kGkMaxWaves && aligned(x, 16) &&
+                     ldx % 8 == 0 && (K * bits / 8) % 16 == 0 && row_bytes % 16 == 0 && aligned(packed, 16);
   // More rows than one k_lowbit_gk (16 bf16) or k_lowbit_slot (5 fp32) launch: one launch over
   // all rows.  17 rows already gain (int3 G = 64: 4096 x 11008 29 -> 17 us, 11008 x 4096
-  // 26 -> 21; int2 G = 64 11008 x 4096 level at 20).
-  if (M > mb && ((scale_dtype == QS_F16 && zeros && zero_dtype == QS_F16) || (scale_dtype == QS_F32 && !zeros))) {
+  // 26 -> 21), except where k_lowbit_gk's blocks of 48 int2 weight rows (G = 64, up to 128
+  // groups) fill most of the chip once: two launches of them, 17 to 32 rows, are the faster
+  // (11008 x 4096 17.4 us against 20.8, x 8192 25.3 against 32.1; 8192 x 4096 17.2 against 16.7
+  // and 14336 x 4096, two rounds of blocks, 29.1 against 23.1).
+  const int64_t gk_blocks = cdiv(N, 48);
+  const bool gk_twice = gk_ok && bits == 2 && group_size == 64 && ng <= kGkMaxWaves * kGkGroupsShort<64> && M <= 32 &&
+                        gk_blocks > 176 && gk_blocks <= 256;
+  if (M > mb && !gk_twice && layout) {
     const LowbitGemm a{x, x_dtype, ldx, packed, row_bytes, scales, zeros, scale_dtype == QS_F16, offset, bits,
                        group_size, y, ldy, M, N, K};
     st = run_lowbit_gemm(a, workspace, workspace_bytes, s);
@@ -1239,7 +1252,6 @@ extern "C" int qs_lowbit_gemv(const void* x, int x_dtype, int64_t ldx, const uin
     int mbv = M <= 1 ? 1 : 2;
     while (mbv > 1 && lds_for(mbv) > kValuLdsMax) mbv /= 2;
     const size_t lds = lds_for(mbv);
-    const bool layout = (scale_dtype == QS_F16 && zeros && zero_dtype == QS_F16) || (scale_dtype == QS_F32 && !zeros);
     const int lb = bits == 3 ? 12 : 16;
     if (x_dtype == QS_BF16 && M <= kValuMaxM && layout && K % cpl == 0 && group_size % cpl == 0 && J <= 6 &&
         J != 5 && row_bytes % lb == 0 && aligned(packed, 16) && aligned(x, 16) && ldx % 8 == 0 &&
@@ -1275,16 +1287,9 @@ extern "C" int qs_lowbit_gemv(const void* x, int x_dtype, int64_t ldx, const uin
     }
   }
   {
-    // 3..16 bf16 rows (and any M that k_lowbit_gemm refuses, in chunks of 16): the
+    // 3..16 bf16 rows (and those k_lowbit_gemm refuses or leaves, in chunks of 16): the
     // single-launch group-MFMA kernel
-    const bool layout = (scale_dtype == QS_F16 && zeros && zero_dtype == QS_F16) || (scale_dtype == QS_F32 && !zeros);
-    const int ngr = group_size == 64 ? kGkGroupsLong<64> : kGkGroupsLong<128>;
-    const int waves = (int)cdiv(ng, ngr);  // the long form's count bounds both
-    const int64_t vb = K * bits / 8;  // code bytes of a row (the kernel reads 16-byte pieces)
-    // scale / zero rows are read as 4-byte words: fp16 arrays need an even group count
-    const bool words = aligned(scales, 4) && (!zeros || aligned(zeros, 4)) && (scale_dtype == QS_F32 || ng % 2 == 0);
-    if (x_dtype == QS_BF16 && layout && words && waves <= kGkMaxWaves && aligned(x, 16) && ldx % 8 == 0 &&
-        vb % 16 == 0 && row_bytes % 16 == 0 && aligned(packed, 16)) {
+    if (gk_ok) {
       LowbitParams p{};
       p.ldx = ldx;
       p.packed = packed;

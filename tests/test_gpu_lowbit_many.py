@@ -49,6 +49,20 @@ def test_many_bf16_rows(dev, bits, G, asym, m, n, k):
     assert oq.rel_l2(y.cpu().numpy(), ref(x)) <= TOL
 
 
+# int2 with G = 64: 17 to 32 rows of widths whose 48-row blocks fill most of the chip once run as
+# two launches of 16 (8449 to 12288 rows), one row more or a narrower or wider block do not.
+@pytest.mark.parametrize("asym", [False, True])
+@pytest.mark.parametrize("m", [17, 32, 33])
+@pytest.mark.parametrize("n", [8448, 8449, 12288, 12289])
+def test_int2_rows_around_the_two_launch_widths(dev, asym, m, n):
+    from mrun_pub_amd.lowbit import lowbit_matmul
+
+    page, ref = _page(2, 64, asym, n, 256, dev, seed=m + n)
+    x = oq.round_bf16(np.random.default_rng(m).standard_normal((m, 256)).astype(np.float32))
+    y = lowbit_matmul(page, torch.from_numpy(x).to(dev).to(torch.bfloat16))
+    assert oq.rel_l2(y.cpu().numpy(), ref(x)) <= TOL
+
+
 @pytest.mark.parametrize("bits,G,asym", [(2, 128, False), (3, 64, True)])
 @pytest.mark.parametrize("m,n,k", [(6, 65, 256), (33, 130, 1024), (515, 40, 256)])
 def test_many_fp32_rows(dev, bits, G, asym, m, n, k):
