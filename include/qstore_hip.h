@@ -148,9 +148,9 @@ int qs_qrow_swiglu(const void* x, int64_t ldx, const int8_t* gate_codes,
  * F32 x) with fp32 sums.  out_indices[m][0..1] (int32) = start_row + row, out_values[m][0..1]
  * the logits: the first is the largest (lowest index on ties), the second the largest of
  * the other rows.  Not bitwise batch invariant: a logit is summed in one order in calls of
- * one or two BF16 / F16 rows (up to four F32) and in another above (aligned rows, K a
- * multiple of 128 from 512), so rows whose candidates nearly tie may order them differently;
- * calls on the same side agree bit for bit.  qs_qrow_rerank_fp32 scores a candidate the same
+ * one or two BF16 / F16 rows (up to four F32; more of a short head) and in another above
+ * (aligned rows, K a multiple of 128 from 512), so rows whose candidates nearly tie may order
+ * them differently; calls on the same side agree bit for bit.  qs_qrow_rerank_fp32 scores a candidate the same
  * way whatever M is.  workspace: qs_qrow_top2_workspace_bytes(M, row_count) bytes of device
  * memory for the per-block candidates.  row_count >= 2. */
 size_t qs_qrow_top2_workspace_bytes(int64_t M, int64_t row_count);

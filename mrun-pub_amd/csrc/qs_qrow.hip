@@ -2137,14 +2137,24 @@ int top2_validate(const void* x, int x_dtype, int64_t ldx, const int8_t* codes, 
   return QS_OK;
 }
 
-// k_head_top2: three or more 16-bit rows (two still fit the register kernel; 151,936 x 1536:
-// two rows 48 us, three 106 -> 59), five or more fp32 rows (four are one VALU launch, 124 us),
-// whose 16-row tile fits LDS.
-bool head_tile_ok(const QrowParams& p, int x_dtype, int64_t M) {
-  const int es = x_dtype == QS_F32 ? 4 : 2;
-  return M >= (x_dtype == QS_F32 ? 5 : 3) && p.K % 128 == 0 && p.K >= 512 &&
-         (int64_t)16 * p.K * es <= 144 * 1024 && p.ldx * es % 16 == 0 && aligned(p.x, 16) &&
-         aligned(p.lin[0].codes, 16);
+// k_head_top2 takes three or more 16-bit rows (two still fit the register kernel; 151,936 x
+// 1536: two rows 48 us, three 106 -> 59), five or more fp32 rows (four are one VALU launch,
+// 124 us), whose 16-row tile fits LDS, where its launches of 16 rows are expected to beat the
+// VALU kernels' of two (fp32: four): a short head leaves a wave one tile, whose chunks of 64 k
+// are a serial chain, and every fp32 tile of a wave is one (us, VALU and this kernel: 512 x
+// 1536, 4 bf16 rows 14.1 and 16.7, 5 rows 19.0 and 16.8; 5 to 17 fp32 rows 16.5 to 35 and 30 to
+// 56; 4096 x 1536, 8 fp32 rows 22 and 32, 16 rows 39 and 32; 8192 x 1024, 4 bf16 rows 19.7 and
+// 16.0).  Times of one launch, in microseconds, fitted to 8 heads of 512 to 50,257 rows.
+bool head_tile_ok(const QrowParams& p, int x_dtype, int64_t M, int rows) {
+  const bool f32 = x_dtype == QS_F32;
+  const int es = f32 ? 4 : 2;
+  if (M < (f32 ? 5 : 3) || p.K % 128 != 0 || p.K < 512 || (int64_t)16 * p.K * es > 144 * 1024 ||
+      p.ldx * es % 16 != 0 || !aligned(p.x, 16) || !aligned(p.lin[0].codes, 16))
+    return false;
+  const float mw = (float)rows * (float)p.K * 1e-6f, chunks = (float)(p.K / 64);
+  const float valu = f32 ? 5.8f + 0.52f * mw : 4.6f + 0.22f * mw;
+  const float tile = f32 ? 6.2f + 0.9f * chunks * (float)cdiv(rows, 16 * 2048) : 5.5f + 0.27f * chunks + 0.1f * mw;
+  return (float)cdiv(M, 16) * tile < (float)cdiv(M, valu_mb(x_dtype, p.K, M)) * valu;
 }
 
 // Workgroups of k_head_top2 (8 waves of 16-row tiles): as many as are resident, two per CU
@@ -2183,7 +2193,7 @@ int top2_launch(const void* x, int x_dtype, int64_t ldx, const int8_t* codes, co
   p.lin[0] = QrowLin{codes, scales, nullptr, 0, (int)row_count, 0};
   const int rows = (int)row_count;
   int C;
-  if (head_tile_ok(p, x_dtype, M)) {
+  if (head_tile_ok(p, x_dtype, M, rows)) {
     const int g = head_grid(rows, (size_t)16 * K * es);  // at most top2_blocks(): the candidates fit the workspace
     C = 2 * g;
     for (int64_t m0 = 0; m0 < M; m0 += 16) {

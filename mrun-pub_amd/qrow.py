@@ -474,8 +474,9 @@ def fused_qrow_top2(
     logits), without materializing logits.  ``require_triton`` and the tile arguments
     keep the reference's signature and checks; the native kernel picks its own tiles.
 
-    Calls of one or two 16-bit rows (up to four fp32) and calls of more rows sum a logit in
-    different orders, so near ties may be ordered differently in a larger batch.
+    Calls of one or two 16-bit rows (up to four fp32, more of a short head) and calls of more
+    rows sum a logit in different orders, so near ties may be ordered differently in a larger
+    batch.
     """
     del require_triton
     _check_head(page, activations)

@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 # 16-row weight tiles (2, 16 and 17 rows), a full wave round of 8 tiles and its remainder,
 # more tiles than the 4096 waves of the largest launch; 8, 10 and 12 chunks of 64 k pick the
 # three windows; 16 activation rows fill the tile, 17 and 33 start another launch.
+# (Fewer rows of the shorter heads take the one- and two-row kernels, fp32 ones up to 17.)
 @pytest.mark.parametrize("v,k", [(2, 512), (16, 640), (17, 768), (129, 1536), (2049, 512), (66000, 512)])
 @pytest.mark.parametrize("m", [3, 5, 16, 17, 33])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
@@ -66,7 +67,7 @@ def test_head_rows_do_not_depend_on_the_batch_within_a_kernel(dev, dtype, few, m
     rerank of given candidates is the same in all."""
     from mrun_pub_amd import qrow as q
 
-    v, k = 4099, 1536
+    v, k = 9001, 768  # long enough that the smallest of `many` takes the many-row kernel
     g = torch.Generator(device=dev).manual_seed(4)
     codes = torch.randint(-127, 128, (v, k), dtype=torch.int8, device=dev, generator=g)
     scales = torch.rand(v, device=dev, generator=g) + 0.5
@@ -89,7 +90,7 @@ def test_head_top2_of_wider_rows(dev, dtype):
     """Activation rows inside wider ones: what lies past k is not read."""
     import mrun_pub_amd._native as nat
 
-    v, k, m, ldx = 300, 640, 19, 640 + 16
+    v, k, m, ldx = 300, 640, 21, 640 + 16
     rng = np.random.default_rng(8)
     codes = rng.integers(-127, 128, size=(v, k), dtype=np.int8)
     scales = np.full(v, 2.0 ** -6, np.float32)
